@@ -43,6 +43,14 @@ inline hipStream_t as_stream(sqx_stream_t s) { return reinterpret_cast<hipStream
 hipError_t int4_gemv_f32out(const uint8_t* wt, const void* st, const void* zt, bool pbf16, const uint16_t* x,
                             float* y, int64_t m, int64_t rows, int64_t cols, int group, hipStream_t s);
 
+// The dequant GEMM of the FP8 linear (sqx_gemm8.hip) on quantized rows: vals [m, cols] the activations' E4M3
+// values as bf16 with per-token scales x_scale [m]; bf16 or (yf32, no bias) fp32 output.
+bool gemm8_fits(int64_t m, int64_t rows, int64_t cols);  // the shape is within the kernel's 32-bit offsets
+int64_t fp8_gemm_workspace_bytes(int64_t m, int64_t rows, int64_t cols);
+hipError_t fp8_gemm(const uint8_t* wt, const float* w_scale, const float* x_scale, const uint16_t* vals, void* y,
+                    bool yf32, const uint16_t* bias, int64_t m, int64_t rows, int64_t cols, float* ws, int64_t ws_bytes,
+                    hipStream_t s);
+
 // ---------------------------------------------------------------- vector types (device) -----
 typedef __bf16 bf16x8_t __attribute__((__vector_size__(8 * sizeof(__bf16))));
 typedef _Float16 f16x8_t __attribute__((__vector_size__(8 * sizeof(_Float16))));
@@ -124,6 +132,11 @@ struct ActBF16 {
   // two floats exactly representable in bf16 -> one bf16 pair (upper halves of the fp32 bits)
   __device__ static inline uint32_t pack_exact(float lo, float hi) {
     return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
+  }
+  // bytes 0,1 (HI false) or 2,3 of d, E4M3 codes, as a bf16 pair (exact for every code)
+  template <bool HI>
+  __device__ static inline uint32_t fp8_pair(uint32_t d) {
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, 1.0f, HI));
   }
   __device__ static inline f32x2_t fp4_pair_f32(uint32_t d, int sel) { return fp4_pair_f32_any(d, sel); }
 
@@ -223,12 +236,20 @@ __device__ inline float ubyte_f32(uint32_t d) {
   return f;
 }
 
-// OCP e4m3fn byte (as quantize_e4m3 values are stored in the tiled NVFP4 scales) -> fp32.
-__device__ inline float e4m3_value(uint32_t b) {
-  const uint32_t e = (b >> 3) & 15u;
-  const uint32_t m = b & 7u;
-  return e ? ldexpf(static_cast<float>(8u + m), static_cast<int>(e) - 10) : ldexpf(static_cast<float>(m), -9);
+// The signed byte SEL of d as fp32 in one instruction.
+template <int SEL>
+__device__ inline float sbyte_f32(uint32_t d) {
+  float f;
+  if (SEL == 0) asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(f) : "v"(d));
+  if (SEL == 1) asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f) : "v"(d));
+  if (SEL == 2) asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(f) : "v"(d));
+  if (SEL == 3) asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(f) : "v"(d));
+  return f;
 }
+
+// OCP e4m3fn byte (as quantize_e4m3 values are stored in the tiled NVFP4 scales) -> fp32: the byte's exponent
+// and mantissa in place in an fp32 are the value times 2**-120 (exact, subnormal codes included).
+__device__ inline float e4m3_value(uint32_t b) { return __builtin_bit_cast(float, (b & 0x7fu) << 20) * 0x1p120f; }
 
 // LDS pointers for the buffer loads that write LDS directly.
 typedef __attribute__((address_space(3))) void lds_void;

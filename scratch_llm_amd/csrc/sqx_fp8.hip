@@ -400,6 +400,9 @@ static SkinnyShape fp8_default_shape(int64_t m, int64_t rows, int64_t cols) {
   return SkinnyShape{0, 2, 8, T >= 256 ? 2 : 4, m <= 16};
 }
 
+// Rows from which sqx_fp8_linear runs the dequant GEMM (the GEMV takes 64 rows per pass over the weight).
+static bool fp8_use_gemm(int64_t m, int64_t rows, int64_t cols) { return m > 64 && gemm8_fits(m, rows, cols); }
+
 static int64_t fp8_ws_bytes(int64_t m, int64_t rows, int64_t cols, const SkinnyShape& sh) {
   if (m <= 0 || rows <= 0 || cols <= 0) return 0;
   const int S = sh.gemv ? 1 : skinny_splits(ceil_div(cols, WFp8::KBLK), sh.S);
@@ -407,7 +410,9 @@ static int64_t fp8_ws_bytes(int64_t m, int64_t rows, int64_t cols, const SkinnyS
 }
 
 extern "C" int64_t sqx_fp8_linear_workspace_bytes(int64_t m, int64_t rows, int64_t cols) {
-  return fp8_ws_bytes(m, rows, cols, fp8_default_shape(m, rows, cols));
+  // the dequant GEMM's partials are optional: without room for them it makes one pass per output tile
+  const int64_t part = fp8_use_gemm(m, rows, cols) ? fp8_gemm_workspace_bytes(m, rows, cols) : 0;
+  return fp8_ws_bytes(m, rows, cols, fp8_default_shape(m, rows, cols)) + part;
 }
 
 extern "C" int64_t sqx_fp8_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits) {
@@ -453,6 +458,10 @@ static int fp8_linear_impl(const uint8_t* wt, const float* w_scale, const void* 
     float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + fp8_part_offset(m, cols));
     e = skinny_launch<ActBF16, WFp8>(a, vals, static_cast<uint16_t*>(y), b16, m, rows, cols, sh, part,
                                      ws_bytes - fp8_part_offset(m, cols), s);
+  } else if (k_slices <= 0 && fp8_use_gemm(m, rows, cols)) {
+    float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + fp8_part_offset(m, cols));
+    e = fp8_gemm(wt, w_scale, xs, vals, y, y_dtype == SQX_DTYPE_F32, b16, m, rows, cols, part,
+                 ws_bytes - fp8_part_offset(m, cols), s);
   } else {
     e = y_dtype == SQX_DTYPE_F32
             ? gemv_launch<ActBF16, WFp8, 4, 2, true>(a, vals, y, b16, nullptr, m, rows, cols, k_slices, s)

@@ -19,15 +19,14 @@
 //
 // Grid order. Workgroups are dispatched round-robin over the 8 XCDs (each with its own L2), so
 // workgroup b runs on XCD b % 8. Each XCD is given a contiguous range of output tiles, walked in
-// groups of kGroupM tile rows, so the workgroups resident on one XCD share X and W fragments in
+// groups of kGemmGroupM tile rows, so the workgroups resident on one XCD share X and W fragments in
 // that XCD's L2.
-#include "sqx_common.h"
+#include "sqx_dqgemm.h"
 
 namespace sqx {
 
 typedef int i32x8_t __attribute__((__vector_size__(8 * sizeof(int))));
 typedef float f32x16_t __attribute__((__vector_size__(16 * sizeof(float))));
-typedef unsigned u32x2_t __attribute__((__vector_size__(2 * sizeof(unsigned))));
 
 namespace mxg {
 constexpr int kTile = 256;                  // output rows and columns per workgroup
@@ -35,22 +34,7 @@ constexpr int kFrags = kTile / 16;          // 16-row fragments per operand per 
 constexpr int kOpBytes = kFrags * 1024;     // one operand's fragments per k-step
 constexpr int kScBytes = kFrags * 64;       // one operand's scale bytes per k-step
 constexpr int kStage = 2 * kOpBytes + 2 * kScBytes;  // X frags | W frags | X scales | W scales
-constexpr int kGroupM = 4;                  // tile rows per group in the walk over output tiles
 }  // namespace mxg
-
-// Output tile (tm, tn) of workgroup `bid`.
-__device__ inline void mx_tile_of(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
-  int lin = bid;
-  if ((total & 7) == 0) lin = (bid & 7) * (total >> 3) + (bid >> 3);  // XCD b % 8 gets a contiguous range
-  const int per_group = mxg::kGroupM * tiles_n;
-  const int g = lin / per_group;
-  const int first_m = g * mxg::kGroupM;
-  const int gm = min(tiles_m - first_m, mxg::kGroupM);
-  const int r = lin - g * per_group;
-  tm = first_m + r % gm;
-  tn = r / gm;
-}
 
 // Issue this wave's share of the global -> LDS copies of k-step kb into `stage`. The 32 fragment
 // copies of a step (16 of X, then 16 of W, 1 KiB per instruction) are split evenly over the NW
@@ -312,393 +296,6 @@ __global__ __launch_bounds__(128 * WN) void mxfp4_gemm_kernel(const uint8_t* __r
 }
 
 
-// ==============================================================================================
-// Dequant GEMM: bf16 / fp16 activations x a tiled 4-bit weight (group INT4 or FP4)
-// ==============================================================================================
-// y[m, n] = sum_k x[m, k] W[n, k] (+ bias[n]) for x [M, K] row-major and W in the tiled layout of
-// sqx_int4.hip (group INT4, symmetric or asymmetric) or sqx_fp4.hip (MXFP4 / NVFP4): the prefill
-// form of w4a16_linear (int4_group.py:148-164), awq_linear (awq.py:184-192) and the config-4
-// FP4-weight linear. Each weight is decoded to the activation dtype in registers exactly as the
-// reference's dequantize(...).to(x.dtype) produces it: INT4 as the fp32 (q - z) * s rounded to
-// nearest even, FP4 as e2m1 * scale (exact; NVFP4's global scale multiplies the fp32 result).
-//
-// Tiling. A workgroup of 8 waves owns a 256 x 256 output tile; wave w computes rows
-// 128 (w / 4) .. +128 and columns 64 (w % 4) .. +64 as 8 x 4 tiles of v_mfma_f32_16x16x32 with the
-// weight as the first operand, so a lane's four accumulators are four consecutive output columns
-// of one row. A stage covers 64 k: the 256 activation rows (32 KiB, 16-byte chunks XOR-swizzled
-// by row so the operand reads of 8 consecutive rows hit distinct banks), the weight bytes of the
-// 16 row tiles for those 64 columns, and their scales; NSTAGE stages form a ring filled by
-// buffer -> LDS copies as in the MXFP4 GEMM. Every wave decodes its own 4 weight tiles per 32-k
-// MFMA step (the decode is shared by the wave's 8 row tiles).
-namespace dqg {
-constexpr int kTile = 256;
-constexpr int kBK = 64;
-constexpr int kXBytes = kTile * kBK * 2;  // activations of one stage
-constexpr int kWBytes = 16 * 512;         // 16 weight row tiles x 512 bytes
-constexpr int kPBytes = 4096;             // scales / zero-points of one stage
-constexpr int kStage = kXBytes + kWBytes + kPBytes;
-constexpr int kStages = 3;
-constexpr int kEpiPitch = 136;            // LDS bytes per row of a wave's 128 x 64 16-bit output tile
-constexpr int kLds = 8 * 128 * kEpiPitch; // 139264 >= kStages * kStage
-static_assert(kStages * kStage <= kLds, "stages fit the LDS allocation");
-}  // namespace dqg
-
-// Weight formats of the dequant GEMM.
-enum : int { kDqInt4 = 0, kDqMx = 1, kDqNv = 2 };
-
-template <int FMT, bool ASYM, bool PBF16, int GROUP>
-struct DqW {
-  // parameter bytes per stage and tile: INT4 scales (and zero-points) of the stage's groups;
-  // MXFP4 32 E8M0 bytes (lanes 32h..32h+31 of the 64-byte block), NVFP4 64 E4M3 bytes
-  // asymmetric bf16 INT4 parameters are (scale, zero) pairs in one dword (sqx_int4_tile)
-  static constexpr bool PAIR = ASYM && PBF16;
-  static constexpr bool ZSEP = ASYM && !PBF16;  // zero-points in a buffer of their own
-  static constexpr int PB = (PBF16 && !PAIR) ? 2 : 4;
-  static constexpr int kWInstr = FMT == kDqInt4 ? 4 : 1;  // weight copies per wave per stage
-  static constexpr int kPInstr = 2;                        // parameter copies per wave per stage
-  static constexpr int NGS = GROUP >= 64 ? 1 : 64 / GROUP;  // INT4 groups per stage
-  static constexpr int NP = FMT == kDqMx ? 2 : FMT == kDqNv ? 4 : (ZSEP ? 2 : 1) * NGS * 16 * 16 * PB / 256;
-  static_assert(NP <= 16, "parameter copies fit two per wave");
-};
-
-template <class A, int FMT, bool ASYM, bool PBF16, int GROUP, int YKIND, int TMR = 256>
-__global__ __launch_bounds__(512) void dq_gemm_kernel(const uint16_t* __restrict__ x, const uint8_t* __restrict__ wt,
-                                                     const void* __restrict__ st, const void* __restrict__ zt,
-                                                     const float* __restrict__ s_global, void* __restrict__ y,
-                                                     const uint16_t* __restrict__ bias, int m, int n, int K, int KB,
-                                                     int tiles_m, int tiles_n, int lds16, int splits,
-                                                     float* __restrict__ ws) {
-  using P = DqW<FMT, ASYM, PBF16, GROUP>;
-  static_assert(TMR == 256 || TMR == 128, "256- or 128-row output tiles");
-  constexpr int group = GROUP;
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  constexpr int NS = dqg::kStages;
-  constexpr int kXI = TMR / 64;   // activation copies per wave per stage (8 rows each)
-  constexpr int RPW = TMR / 8;    // activation rows a wave copies
-  constexpr int MT = TMR / 32;    // 16-row MFMA tiles of a wave (it owns TMR / 2 rows)
-  constexpr int kPerStage = kXI + P::kWInstr + P::kPInstr;  // buffer -> LDS copies per wave per stage
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int tm, tn;
-  // split-K: workgroup b computes split b % splits of tile b / splits (stages s0 .. s0+S-1)
-  const int tile = blockIdx.x / splits, split = blockIdx.x - tile * splits;
-  mx_tile_of(tile, tiles_m, tiles_n, tm, tn);
-  const int S_all = 2 * KB;  // stages of 64 columns (the tiled weight is padded to 128-column blocks)
-  const int Sp = (S_all + splits - 1) / splits;
-  const int s0 = split * Sp;
-  const int S = min(S_all, s0 + Sp) - s0;
-  const int wT = (n + 15) >> 4;
-  const int w_t0 = tn * 16;
-  const int Gp = KB * (128 / (FMT == kDqInt4 ? GROUP : 128));  // INT4 groups per row (padded)
-
-  const rsrc_t xr = make_rsrc(x, (uint32_t)((uint64_t)m * (uint64_t)K * 2u));
-  const rsrc_t wr = make_rsrc(wt, (uint32_t)wT * (uint32_t)KB * 1024u);
-  uint32_t pbytes;
-  if (FMT == kDqInt4) pbytes = (uint32_t)wT * (uint32_t)Gp * 16u * P::PB;
-  else pbytes = (uint32_t)wT * (uint32_t)KB * (FMT == kDqMx ? 64u : 128u);
-  const rsrc_t sr = make_rsrc(st, pbytes);
-  const rsrc_t zr = make_rsrc(ASYM ? zt : st, pbytes);
-  constexpr int np = P::NP;
-
-  // ---- copies of stage s into ring slot `slot`
-  auto issue = [&](int s, int slot) {
-    uint8_t* base = smem + slot * dqg::kStage;
-    const int kb = s >> 1, h = s & 1;
-    // activations: wave w copies rows RPW*w .. RPW*w + RPW-1 (8 rows of 8 chunks per instruction)
-#pragma unroll
-    for (int j = 0; j < kXI; ++j) {
-      const int r = RPW * wave + 8 * j + (lane >> 3);
-      const int c = (lane & 7) ^ (r & 7);
-      const int R = tm * TMR + r, col = 64 * s + 8 * c;
-      const bool ok = (R < m) & (col < K);  // no short-circuit: a select, not a branch
-      const uint32_t off = ok ? ((uint32_t)R * (uint32_t)K + (uint32_t)col) * 2u : 0xFFFFFFF0u;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(base + (RPW * wave + 8 * j) * 128), 16, off, 0, 0, 0);
-    }
-    uint8_t* wbase = base + dqg::kXBytes;
-    if (FMT == kDqInt4) {
-      // tiles 2w, 2w+1: dwords 2h and 2h+1 of every lane's 16 bytes, 256 bytes per copy
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int f = 2 * wave + (j >> 1), i = 2 * h + (j & 1);
-        const int t = min(w_t0 + f, wT - 1);
-        const uint32_t off = ((uint32_t)t * (uint32_t)KB + (uint32_t)kb) * 1024u + (uint32_t)lane * 16u + (uint32_t)i * 4u;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(wbase + f * 512 + (j & 1) * 256), 4, off, 0, 0, 0);
-      }
-    } else {
-      // tiles 2w (lanes 0-31) and 2w+1 (lanes 32-63): bytes 512h .. 512h+511 of their blocks
-      const int f = 2 * wave + (lane >> 5);
-      const int t = min(w_t0 + f, wT - 1);
-      const uint32_t off = ((uint32_t)t * (uint32_t)KB + (uint32_t)kb) * 1024u + 512u * (uint32_t)h + (uint32_t)(lane & 31) * 16u;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(wbase + 2 * wave * 512), 16, off, 0, 0, 0);
-    }
-    uint8_t* pbase = base + dqg::kXBytes + dqg::kWBytes;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int pi = 2 * wave + j;  // parameter copy index; copies past np land in unused LDS
-      const int pr = pi < np ? pi : 0;
-      uint32_t off;
-      bool zsrc = false;
-      if (FMT == kDqInt4) {
-        // layout in LDS: [scales | zeros][group gi][tile f][row] of PB bytes; 256 bytes per copy
-        constexpr int TPI = 256 / (16 * P::PB);  // tiles per copy
-        const int per_kind = np / (P::ZSEP ? 2 : 1);
-        zsrc = P::ZSEP && pr >= per_kind;
-        const int q = pr - (zsrc ? per_kind : 0);
-        const int gi = q / (16 / TPI);
-        const int f = TPI * (q % (16 / TPI)) + lane / (64 / TPI);
-        const int t = min(w_t0 + f, wT - 1);
-        const int g = (64 * s) / group + gi;
-        off = ((uint32_t)t * (uint32_t)Gp + (uint32_t)g) * 16u * P::PB + (uint32_t)(lane % (64 / TPI)) * 4u;
-      } else if (FMT == kDqMx) {
-        const int f = 8 * pr + (lane >> 3);
-        const int t = min(w_t0 + f, wT - 1);
-        off = ((uint32_t)t * (uint32_t)KB + (uint32_t)kb) * 64u + 32u * (uint32_t)h + (uint32_t)(lane & 7) * 4u;
-      } else {
-        const int f = 4 * pr + (lane >> 4);
-        const int t = min(w_t0 + f, wT - 1);
-        off = ((uint32_t)t * (uint32_t)KB + (uint32_t)kb) * 128u + 64u * (uint32_t)h + (uint32_t)(lane & 15) * 4u;
-      }
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(zsrc ? zr : sr, (lds_void*)(pbase + pi * 256), 4, off, 0, 0, 0);
-    }
-  };
-
-  f32x4_t acc[MT][4];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int wm = wave >> 2, wn = wave & 3;
-  const int nl = lane & 15, jg = lane >> 4;
-  // p0: the scale's fp32 bits, or for bf16 INT4 parameters bf16 scale | bf16 zero-point << 16;
-  // p1: fp32 zero-points (asymmetric INT4 with fp32 parameters only)
-  constexpr int kP1 = (FMT == kDqInt4 && ASYM && !PBF16) ? 4 : 1;
-  struct Raw {
-    u32x4_t xo[MT];  // activation operands of the wave's row tiles
-    uint32_t wd[4];  // weight codes of the 4 column tiles
-    uint32_t p0[4], p1[kP1];
-  };
-  // operands of MFMA step q (32 columns) of the stage in ring slot `slot`
-  auto read = [&](int slot, int s, int q, Raw& o) {
-    const uint8_t* base = smem + slot * dqg::kStage;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int r = wm * (TMR / 2) + 16 * mt + nl;
-      const int sl = (4 * q + jg) ^ (nl & 7);
-      o.xo[mt] = *reinterpret_cast<const u32x4_t*>(base + r * 128 + sl * 16);
-    }
-    const uint8_t* wb = base + dqg::kXBytes;
-    const uint8_t* pb = base + dqg::kXBytes + dqg::kWBytes;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int f = wn * 4 + nt;
-      if (FMT == kDqInt4) {
-        o.wd[nt] = *reinterpret_cast<const uint32_t*>(wb + f * 512 + q * 256 + lane * 4);
-        const int gi = GROUP >= 64 ? 0 : (32 * q) / GROUP;
-        constexpr int zoff = P::NGS * 16 * 16 * P::PB;
-        const int po = ((gi * 16 + f) * 16 + nl) * P::PB;
-        if (P::PAIR) {
-          o.p0[nt] = *reinterpret_cast<const uint32_t*>(pb + po);  // bf16 scale | bf16 zero << 16
-        } else if (PBF16) {
-          o.p0[nt] = *reinterpret_cast<const uint16_t*>(pb + po);
-        } else {
-          o.p0[nt] = *reinterpret_cast<const uint32_t*>(pb + po);
-          if (ASYM) o.p1[nt % kP1] = *reinterpret_cast<const uint32_t*>(pb + zoff + po);
-        }
-      } else {
-        const int ll = 16 * q + nl;  // lane of the 128-column block within the stage's half
-        o.wd[nt] = *reinterpret_cast<const uint32_t*>(wb + f * 512 + ll * 16 + jg * 4);
-        if (FMT == kDqMx) {
-          o.p0[nt] = (uint32_t)pb[f * 32 + ll] << 23;  // the fp32 2**(e - 127)
-        } else {
-          o.p0[nt] = __builtin_bit_cast(uint32_t, e4m3_value(pb[f * 64 + 2 * ll + (jg >> 1)]));
-        }
-      }
-    }
-    (void)s;
-  };
-  // weight operand of column tile nt: 8 consecutive k of row nl, in the activation dtype
-  auto decode = [&](const Raw& o, int nt) -> u32x4_t {
-    const uint32_t d = o.wd[nt];
-    if (FMT == kDqMx) {
-      const float sc = __builtin_bit_cast(float, o.p0[nt]);
-      return u32x4_t{A::fp4_pair_scaled(d, sc, 0), A::fp4_pair_scaled(d, sc, 1), A::fp4_pair_scaled(d, sc, 2),
-                     A::fp4_pair_scaled(d, sc, 3)};
-    }
-    float w[8];
-    if (FMT == kDqNv) {
-      const float sc = __builtin_bit_cast(float, o.p0[nt]);
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const f32x2_t f = A::fp4_pair_f32(d, p);
-        w[2 * p] = f[0] * sc;
-        w[2 * p + 1] = f[1] * sc;
-      }
-      return u32x4_t{A::pack_exact(w[0], w[1]), A::pack_exact(w[2], w[3]), A::pack_exact(w[4], w[5]),
-                     A::pack_exact(w[6], w[7])};
-    }
-    // INT4: element e in nibble e/2 (even e) or 4 + e/2 (odd e); u as fp32, then fp32 (u - z) * s
-    const uint32_t lo = d & 0x0F0F0F0Fu, hi = (d >> 4) & 0x0F0F0F0Fu;
-    const float u[8] = {ubyte_f32<0>(lo), ubyte_f32<2>(lo), ubyte_f32<0>(hi), ubyte_f32<2>(hi),
-                        ubyte_f32<1>(lo), ubyte_f32<3>(lo), ubyte_f32<1>(hi), ubyte_f32<3>(hi)};
-    const float sc = PBF16 ? bf16_bits_to_f32((uint16_t)(o.p0[nt] & 0xffffu)) : __builtin_bit_cast(float, o.p0[nt]);
-    if (!ASYM || PBF16) {
-      // z * s is exact (z = 8, or z <= 15 and s has at most 8 significant bits), so the fma rounds
-      // the exact (u - z) * s once
-      const float zf = ASYM ? bf16_bits_to_f32((uint16_t)(o.p0[nt] >> 16)) : 8.0f;
-      const float c = -zf * sc;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) w[e] = fmaf(u[e], sc, c);
-    } else {
-      const float zf = __builtin_bit_cast(float, o.p1[nt % kP1]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) w[e] = (u[e] - zf) * sc;
-    }
-    return u32x4_t{A::pack_rne(w[0], w[1]), A::pack_rne(w[2], w[3]), A::pack_rne(w[4], w[5]), A::pack_rne(w[6], w[7])};
-  };
-  auto mma = [&](const Raw& o) {
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const u32x4_t b = decode(o, nt);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = A::mfma(b, o.xo[mt], acc[mt][nt]);
-    }
-  };
-
-  // pipeline (as the MXFP4 GEMM): iteration s: read (s, 1) | MFMAs (s, 0) | wait for stage s+1,
-  // barrier | copy stage s+NS-1 into the slot of s-1 | read (s+1, 0) | MFMAs (s, 1)
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < S) issue(s0 + s, s);
-  if (S - 1 >= NS - 2) wait_vmcnt<kPerStage * (NS - 2)>();
-  else wait_vmcnt<0>();
-  __builtin_amdgcn_s_barrier();
-  Raw o0, o1;
-  read(0, 0, 0, o0);
-  int s = 0;
-  for (; s + NS - 1 < S; ++s) {
-    read(s % NS, s, 1, o1);
-    mma(o0);
-    __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<kPerStage * (NS - 3)>();
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    issue(s0 + s + NS - 1, (s + NS - 1) % NS);
-    read((s + 1) % NS, s + 1, 0, o0);
-    mma(o1);
-  }
-  for (; s < S; ++s) {
-    read(s % NS, s, 1, o1);
-    mma(o0);
-    __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + 1 < S) read((s + 1) % NS, s + 1, 0, o0);
-    mma(o1);
-  }
-
-  // epilogue: acc[mt][nt][i] is y[m0 + 16mt + (l & 15)][n0 + 16nt + 4(l >> 4) + i]
-  const int m0 = tm * TMR + wm * (TMR / 2);
-  const int n0 = tn * dqg::kTile + wn * 64;
-  if (splits > 1) {
-    // raw fp32 partial sums of this split; dq_reduce_kernel adds the splits in order
-    float* part = ws + (int64_t)split * m * n;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int col = n0 + 16 * nt + 4 * jg;
-      if (col >= n) continue;
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int row = m0 + 16 * mt + nl;
-        if (row >= m) continue;
-        float* dst = part + (int64_t)row * n + col;
-        if ((n & 3) == 0) {
-          *reinterpret_cast<f32x4_t*>(dst) = acc[mt][nt];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (col + j < n) dst[j] = acc[mt][nt][j];
-        }
-      }
-    }
-    return;
-  }
-  const float gs = FMT == kDqNv ? *s_global : 1.0f;
-  if (YKIND != 2 && lds16) {
-    __builtin_amdgcn_s_barrier();  // every wave is done reading the stages
-    uint8_t* ep = smem + wave * 128 * dqg::kEpiPitch;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int cl = 16 * nt + 4 * jg;
-      float badd[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (bias) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (n0 + cl + j < n) badd[j] = YKIND == 1 ? f16_bits_to_f32(bias[n0 + cl + j]) : bf16_bits_to_f32(bias[n0 + cl + j]);
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int rl = 16 * mt + nl;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = acc[mt][nt][j] * gs + badd[j];
-        const uint32_t lo = YKIND == 0 ? ActBF16::pack_rne(v[0], v[1]) : ActF16::pack_rne(v[0], v[1]);
-        const uint32_t hi = YKIND == 0 ? ActBF16::pack_rne(v[2], v[3]) : ActF16::pack_rne(v[2], v[3]);
-        *reinterpret_cast<u32x2_t*>(ep + rl * dqg::kEpiPitch + cl * 2) = u32x2_t{lo, hi};
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    const int cc = (lane & 7) * 8;
-#pragma unroll 4
-    for (int p = 0; p < TMR / 16; ++p) {
-      const int rl = 8 * p + (lane >> 3);
-      const int row = m0 + rl, col = n0 + cc;
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ep + rl * dqg::kEpiPitch + cc * 2);
-      if (row >= m || col >= n) continue;
-      uint16_t* dst = static_cast<uint16_t*>(y) + (int64_t)row * n + col;
-      __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(dst));
-    }
-    return;
-  }
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int col = n0 + 16 * nt + 4 * jg;
-    if (col >= n) continue;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int row = m0 + 16 * mt + nl;
-      if (row >= m) continue;
-      const int64_t o = (int64_t)row * n + col;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (col + j >= n) break;
-        float v = acc[mt][nt][j] * gs;
-        if (bias) v += YKIND == 1 ? f16_bits_to_f32(bias[col + j]) : bf16_bits_to_f32(bias[col + j]);
-        if (YKIND == 0) static_cast<uint16_t*>(y)[o + j] = f32_to_bf16_bits(v);
-        else if (YKIND == 1) static_cast<uint16_t*>(y)[o + j] = f32_to_f16_bits(v);
-        else static_cast<float*>(y)[o + j] = v;
-      }
-    }
-  }
-}
-
-// y[i] = (sum over splits, in order, of the fp32 partials) * gs (+ bias[i % n]), rounded to y's dtype.
-template <int YKIND>
-__global__ __launch_bounds__(256) void dq_reduce_kernel(const float* __restrict__ ws, int splits, int64_t mn, int n,
-                                                        const float* __restrict__ s_global,
-                                                        const uint16_t* __restrict__ bias, void* __restrict__ y) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= mn) return;
-  float v = 0.0f;
-  for (int s = 0; s < splits; ++s) v += ws[(int64_t)s * mn + i];
-  if (s_global) v *= *s_global;
-  if (bias) v += YKIND == 1 ? f16_bits_to_f32(bias[i % n]) : bf16_bits_to_f32(bias[i % n]);
-  if (YKIND == 0) static_cast<uint16_t*>(y)[i] = f32_to_bf16_bits(v);
-  else if (YKIND == 1) static_cast<uint16_t*>(y)[i] = f32_to_f16_bits(v);
-  else static_cast<float*>(y)[i] = v;
-}
-
 }  // namespace sqx
 
 using namespace sqx;
@@ -761,8 +358,9 @@ hipError_t launch_mx(const uint8_t* xt, const uint8_t* xst, const uint8_t* wt, c
                      (int64_t)m * n);
   if (splits > 1) {
     const int64_t mn = (int64_t)m * n;
-    hipLaunchKernelGGL(dq_reduce_kernel<YK>, dim3((unsigned)ceil_div(mn, 256)), dim3(256), 0, s, ws, splits, mn, n,
-                       nullptr, bias, y);
+    const int v4 = n % 4 == 0 && reinterpret_cast<uintptr_t>(y) % (YK == 2 ? 16 : 8) == 0;
+    hipLaunchKernelGGL(dq_reduce_kernel<YK>, dim3((unsigned)ceil_div(mn, v4 ? 1024 : 256)), dim3(256), 0, s, ws, splits,
+                       mn, n, nullptr, nullptr, nullptr, bias, y, v4);
   }
   return hipGetLastError();
 }
@@ -845,57 +443,44 @@ extern "C" int sqx_mxfp4_gemm_ws(const uint8_t* xt, const uint8_t* xst, const ui
                 as_stream(stream));
 }
 
-namespace {
-// K splits for a shape: when the output tiles fill less than three quarters of the 256 CUs, as many
-// splits as keep the workgroups within one round on the CUs (a second, partial round costs more than
-// the splits save, and every split adds M x N fp32 partials to write and reduce), at least 4 stages
-// (256 columns) per split, and no empty split.
-// Output-tile rows: 128 for M <= 128, where a 256-row tile is at least half padding (config 4's
-// bf16 activations at M = 128: 106 -> 74 us and 96 -> 65 us), else 256: a 128-row tile decodes each
-// weight for half as many MFMAs, and at M = 512 / 2048 it measured slower on the 14336-wide shapes
-// (97 -> 104 us, 298 -> 364 us) and within 6 % elsewhere. Also 128 when 256-row tiles would number
-// fewer than 16, where the K splits that fill the CUs are the cost (4096->1024 at M = 512, which
-// splits 16 ways either way: 31.9 -> 28.3 us; 4096x4096 at M = 512 has 32 tiles: 44.3 us against
-// 43.0 us at its best 128-row split, so it stays).
-int dq_tile_rows(int64_t m, int64_t rows) {
-  if (m <= 128) return 128;
-  return ceil_div(m, 256) * ceil_div(rows, dqg::kTile) < 16 ? 128 : 256;
-}
-
-int dq_splits(int64_t m, int64_t rows, int64_t cols) {
-  const int64_t tiles = ceil_div(m, dq_tile_rows(m, rows)) * ceil_div(rows, dqg::kTile);
-  const int64_t S = 2 * ceil_div(cols, 128);
-  if (tiles >= 192) return 1;
-  const int64_t want = std::min<int64_t>(std::min<int64_t>(256 / tiles, S / 4), 16);
-  if (want < 2) return 1;
-  const int64_t per = ceil_div(S, want);
-  return (int)ceil_div(S, per);
-}
-
-template <class A, int FMT, bool ASYM, bool PBF16, int GROUP, int YK>
-hipError_t launch_dq(const uint16_t* x, const uint8_t* wt, const void* st, const void* zt, const float* s_global,
-                     void* y, const uint16_t* bias, int m, int n, int K, int KB, float* ws, int64_t ws_bytes,
-                     hipStream_t s) {
-  const int tmr = dq_tile_rows(m, n);
-  const int tiles_m = (m + tmr - 1) / tmr, tiles_n = (n + dqg::kTile - 1) / dqg::kTile;
-  int splits = dq_splits(m, n, K);
-  if (splits > 1 && (ws == nullptr || ws_bytes < (int64_t)splits * m * n * 4 || reinterpret_cast<uintptr_t>(ws) % 16))
-    splits = 1;  // no (or too small a) workspace: one pass per tile
-  auto kern = tmr == 128 ? dq_gemm_kernel<A, FMT, ASYM, PBF16, GROUP, YK, 128> : dq_gemm_kernel<A, FMT, ASYM, PBF16, GROUP, YK, 256>;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     dqg::kLds);
-  if (e != hipSuccess) return e;
-  const int lds16 = YK != 2 && (n % 8 == 0) && (reinterpret_cast<uintptr_t>(y) % 16 == 0);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(512), dqg::kLds, s, x, wt, st, zt,
-                     s_global, y, bias, m, n, K, KB, tiles_m, tiles_n, lds16, splits, ws);
-  if (splits > 1) {
-    const int64_t mn = (int64_t)m * n;
-    hipLaunchKernelGGL(dq_reduce_kernel<YK>, dim3((unsigned)ceil_div(mn, 256)), dim3(256), 0, s, ws, splits, mn, n,
-                       FMT == kDqNv ? s_global : nullptr, bias, y);
+// Output tile and K splits of the dequant GEMM, the cheapest under a cost model fitted to a sweep of 65..2048
+// rows at the Llama-3-8B shapes (int8, MXFP4, symmetric and asymmetric int4; every tile with every split).
+// A workgroup fills a CU (its stages take 110 to 150 KiB of LDS), so tiles * S workgroups run in
+// ceil(tiles * S / 256) rounds of ceil(stages / S) stages, plus about 4 us of launch, prologue and epilogue.
+// A stage takes, with a share b of the CUs busy (us):
+//                8-bit           FP4             int4
+//   256 x 256    0.85 + 0.70 b   0.97 + 0.45 b   1.45 + 0.40 b   the fewest bytes and decodes per MFMA
+//   128 x 256    0.68 + 0.30 b   0.70 + 0.18 b   0.95 + 0.30 b
+//   128 x 128    0.47 + 0.12 b   0.57 + 0.03 b   0.67 + 0.06 b   short m or narrow n
+// (int8 4096 -> 4096 at 1000 rows: 42 us on 128 x 128 tiles, 55 us on 256 x 256 in four splits). K splits add
+// 3 us for the reduce launch and 8 bytes per output and split at about 5 TB/s.
+DqPlan sqx::dq_plan(int64_t m, int64_t rows, int64_t stages, int fmt) {
+  struct Tile {
+    int tm, tn;
+    double idle[3], busy[3];
+  };
+  static constexpr Tile kTiles[] = {{256, 256, {0.85, 0.97, 1.45}, {0.70, 0.45, 0.40}},
+                                    {128, 256, {0.68, 0.70, 0.95}, {0.30, 0.18, 0.30}},
+                                    {128, 128, {0.47, 0.57, 0.67}, {0.12, 0.03, 0.06}}};
+  const int f = fmt == kDqInt4 ? 2 : fmt == kDqMx || fmt == kDqNv ? 1 : 0;
+  DqPlan best{256, 256, 1};
+  double best_us = 0.0;
+  bool first = true;
+  for (const auto& t : kTiles) {
+    const int64_t tiles = ceil_div(m, t.tm) * ceil_div(rows, t.tn);
+    for (int S = 1; S <= 16 && (S == 1 || (S <= stages / 4 && tiles * S <= 256)); ++S) {
+      const int64_t per = ceil_div(stages, S), wgs = tiles * S;
+      if (ceil_div(stages, per) != S) continue;  // the last split would be empty
+      const double b = wgs >= 256 ? 1.0 : (double)wgs / 256.0;
+      double us = 4.0 + (double)ceil_div(wgs, 256) * (double)per * (t.idle[f] + t.busy[f] * b);
+      if (S > 1) us += 3.0 + (double)S * (double)m * (double)rows * 8.0 / 5e6;
+      if (first || us < best_us) best = DqPlan{t.tm, t.tn, S}, best_us = us, first = false;
+    }
   }
-  return hipGetLastError();
+  return best;
 }
 
+namespace {
 // shape checks shared by the dequant GEMM entry points
 int dq_check(const char* fn, const void* x, const void* wt, const void* y, int64_t m, int64_t rows, int64_t cols) {
   SQX_REQUIRE(m >= 0 && rows > 0 && cols > 0 && cols % 32 == 0, SQX_E_ARG,
@@ -913,8 +498,9 @@ int dq_check(const char* fn, const void* x, const void* wt, const void* y, int64
 
 extern "C" int64_t sqx_gemm_workspace_bytes(int64_t m, int64_t rows, int64_t cols) {
   if (m <= 0 || rows <= 0 || cols <= 0) return 0;
-  const int sp = dq_splits(m, rows, cols);
-  return sp > 1 ? (int64_t)sp * m * rows * 4 : 0;
+  const int64_t stages = 2 * ceil_div(cols, 128);  // int4 and FP4 plans differ: room for either
+  return std::max(dq_workspace_bytes(dq_plan(m, rows, stages, kDqInt4), m, rows),
+                  dq_workspace_bytes(dq_plan(m, rows, stages, kDqMx), m, rows));
 }
 
 extern "C" int sqx_int4_gemm(const uint8_t* wt, const void* st, const void* zt, int param_dtype, const void* x,
@@ -938,7 +524,7 @@ extern "C" int sqx_int4_gemm(const uint8_t* wt, const void* st, const void* zt, 
   hipStream_t s = as_stream(stream);
   hipError_t e;
 #define SQX_DQG(ACT, AS, PB, G, YK) \
-  e = launch_dq<ACT, kDqInt4, AS, PB, G, YK>(xp, wt, st, zt, nullptr, y, b16, (int)m, (int)rows, (int)cols, KB, \
+  e = launch_dq<ACT, kDqInt4, AS, PB, G, YK>(xp, wt, st, zt, nullptr, nullptr, y, b16, (int)m, (int)rows, (int)cols, KB, \
                                              static_cast<float*>(ws), ws_bytes, s)
 #define SQX_DQ(ACT, AS, PB, YK)                               \
   do {                                                        \
@@ -978,7 +564,7 @@ extern "C" int sqx_fp4_gemm(const uint8_t* wt, const uint8_t* st, int fmt, const
   const bool yf = y_dtype == SQX_DTYPE_F32;
   hipError_t e;
 #define SQX_DQ(ACT, F, YK) \
-  e = launch_dq<ACT, F, false, false, 128, YK>(xp, wt, st, nullptr, s_global, y, b16, (int)m, (int)rows, (int)cols, KB, \
+  e = launch_dq<ACT, F, false, false, 128, YK>(xp, wt, st, nullptr, s_global, nullptr, y, b16, (int)m, (int)rows, (int)cols, KB, \
                                               static_cast<float*>(ws), ws_bytes, s)
   if (act_dtype == SQX_DTYPE_BF16) {
     if (fmt == SQX_FP4_MX) { if (yf) SQX_DQ(ActBF16, kDqMx, 2); else SQX_DQ(ActBF16, kDqMx, 0); }
