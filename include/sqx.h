@@ -440,6 +440,15 @@ int sqx_e2m1_round_rne(const double* v, int64_t n, uint8_t* codes, int* status, 
 int sqx_fp4_linear(const uint8_t* wt, const uint8_t* st, int fmt, const float* s_global, const void* x,
                    int act_dtype, void* y, int y_dtype, const void* bias, int64_t m, int64_t rows,
                    int64_t cols, int k_slices, sqx_stream_t stream);
+/* The same product for 1..64 rows with y in act_dtype on the row-tiled decode kernels (as sqx_int4_skinny):
+ * variant 0 = waves splitting K (tiles 2 or 4, waves 1..8), 1 = activations staged through LDS (tiles 1, 2 or
+ * 4, waves 4 or 8), splits workgroups along K (fp32 partials in ws, added in split order); -1 / 0 = the
+ * library's choice, the GEMV included. ws: sqx_fp4_skinny_workspace_bytes(m, rows, cols, splits) bytes. */
+int64_t sqx_fp4_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits);
+int sqx_fp4_skinny(const uint8_t* wt, const uint8_t* st, int fmt, const float* s_global, const void* x,
+                   int act_dtype, void* y, const void* bias, int64_t m, int64_t rows, int64_t cols, int variant,
+                   int tiles, int waves, int splits, void* ws, int64_t ws_bytes, sqx_stream_t stream);
+
 
 /* mxfp4_quantize (nvfp4_mxfp4.py:257-265, block 32) of each row of x [m, k] (k a multiple of 32, so
  * every block lies in one row), written in the tiled FP4 layout sqx_fp4_tile produces: xt
@@ -570,6 +579,13 @@ int sqx_int8_untile(const uint8_t* wt, int64_t rows, int64_t cols, int8_t* q, sq
 int sqx_int8_linear(const uint8_t* wt, const float* scale, const void* x, int act_dtype, void* y,
                     const void* bias, int64_t m, int64_t rows, int64_t cols, int k_slices,
                     sqx_stream_t stream);
+/* The same product for 1..64 rows on the row-tiled decode kernel (waves splitting K): tiles (2 or 4) of 16 rows
+ * per workgroup, waves 1..8, splits workgroups along K (fp32 partials in ws, added in split order); all 0 = the
+ * library's choice, the GEMV included. ws: sqx_int8_skinny_workspace_bytes(m, rows, cols, splits) bytes. */
+int64_t sqx_int8_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits);
+int sqx_int8_skinny(const uint8_t* wt, const float* scale, const void* x, int act_dtype, void* y, const void* bias,
+                    int64_t m, int64_t rows, int64_t cols, int tiles, int waves, int splits, void* ws,
+                    int64_t ws_bytes, sqx_stream_t stream);
 /* The same product from 65 rows on (prefill): the dequant GEMM on the tiled int8 weight, whose codes are
  * exact in the activation dtype, with the per-row scale on the fp32 sum. cols % 8 == 0; ws: at least
  * sqx_int8_gemm_workspace_bytes(m, rows, cols) bytes, 16-byte aligned, for the fp32 partials of the K splits

@@ -124,6 +124,11 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _c_i,
         [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p],
     ),
+    "sqx_fp4_skinny_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i]),
+    "sqx_fp4_skinny": (
+        _c_i,
+        [_c_p, _c_p, _c_i, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_i, _c_i, _c_i, _c_p, _c_i64, _c_p],
+    ),
     "sqx_fp4_gemm": (
         _c_i,
         [_c_p, _c_p, _c_i, _c_p, _c_p, _c_i, _c_p, _c_i, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p],
@@ -146,6 +151,9 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "sqx_int8_tiled_weight_bytes": (_c_i64, [_c_i64, _c_i64]),
     "sqx_int8_tile": (_c_i, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),
     "sqx_int8_linear": (_c_i, [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_p]),
+    "sqx_int8_skinny_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i]),
+    "sqx_int8_skinny": (_c_i, [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_i, _c_i, _c_p, _c_i64,
+                               _c_p]),
     "sqx_int8_gemm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "sqx_int8_gemm": (_c_i, [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p]),
     "sqx_int4_quantize_asym": (_c_i, [_c_p, _c_i, _c_i64, _c_i64, _c_i64, _c_i, _c_p, _c_p, _c_p, _c_p]),

@@ -9,7 +9,7 @@
 // reference's row-major packed weight. Scales per block (t, kb): MXFP4 64 bytes, byte L the E8M0
 // scale of lane L's 32 columns; NVFP4 128 bytes, bytes 2L and 2L+1 the E4M3 scales of lane L's two
 // 16-column halves. Padding rows / columns hold code 0 and scale byte 0.
-#include "sqx_gemv.h"
+#include "sqx_skinny.h"
 #include "sqx_mx.h"
 
 #include <float.h>
@@ -415,53 +415,65 @@ struct WFp4 {
     uint32_t wvo, svo;
   };
   struct P {
-    float s0, s1;
+    uint32_t raw;  // the scale byte(s) as loaded: a conversion here would wait for the load
+    __device__ float scale(int i) const {  // of MFMA step i's columns
+      if (NV) return e4m3_value(i < 2 ? raw & 0xffu : raw >> 8);
+      // E8M0 byte e -> the fp32 2**(e-127) (the conversion uses only the scale's exponent field)
+      return __builtin_bit_cast(float, raw << 23);
+    }
   };
-  __device__ static Ctx ctx(const Args& a, int t, int KB, int lane) {
+  __device__ static Ctx ctx(const Args& a, int t, int KB, int lane) { return ctx_tiles(a, t, 1, KB, lane); }
+  // tiles t .. t+nt-1, contiguous in HBM: block kb of tile r is block r*KB + kb
+  __device__ static Ctx ctx_tiles(const Args& a, int t, int nt, int KB, int lane) {
     Ctx c;
-    c.wr = make_rsrc(a.wt + (int64_t)t * KB * 1024, (uint32_t)KB * 1024u);
+    c.wr = make_rsrc(a.wt + (int64_t)t * KB * 1024, (uint32_t)nt * (uint32_t)KB * 1024u);
     const uint32_t sbytes = (uint32_t)KB * (NV ? 128u : 64u);
-    c.sr = make_rsrc(a.st + (int64_t)t * sbytes, sbytes);
+    c.sr = make_rsrc(a.st + (int64_t)t * sbytes, (uint32_t)nt * sbytes);
     c.wvo = (uint32_t)lane * 16u;
     c.svo = (uint32_t)lane * (NV ? 2u : 1u);
     return c;
   }
   __device__ static void load(const Ctx& c, int kb, u32x4_t& w, P& p) {
     w = bload128<2>(c.wr, c.wvo, (uint32_t)kb * 1024u);
-    if (NV) {
-      const uint32_t b = bload16(c.sr, c.svo, (uint32_t)kb * 128u);
-      p.s0 = e4m3_value(b & 0xffu);
-      p.s1 = e4m3_value(b >> 8);
-    } else {
-      // E8M0 byte e -> the fp32 2**(e-127) (the conversion uses only the scale's exponent field)
-      p.s0 = __builtin_bit_cast(float, bload8(c.sr, c.svo, (uint32_t)kb * 64u) << 23);
-      p.s1 = p.s0;
-    }
+    p.raw = NV ? bload16(c.sr, c.svo, (uint32_t)kb * 128u) : bload8(c.sr, c.svo, (uint32_t)kb * 64u);
   }
   __device__ static int xk(int i, int jg) { return 32 * jg + 8 * i; }
+  // B fragment of step i: the weights themselves (NVFP4: times its E4M3 block scale; E4M3 scales carry
+  // mantissa bits, so decode to fp32, scale, pack: e2m1 * s_b has <= 6 significant bits, exact in bf16 / fp16)
+  template <class A>
+  __device__ static u32x4_t bfrag(const u32x4_t& w, const P& p, int i) {
+    const uint32_t d = w[i];
+    const float s = p.scale(i);
+    u32x4_t b;
+#pragma unroll
+    for (int sel = 0; sel < 4; ++sel) {
+      if (NV) {
+        const f32x2_t f = A::fp4_pair_f32(d, sel);
+        b[sel] = A::pack_exact(f[0] * s, f[1] * s);
+      } else {
+        b[sel] = A::fp4_pair_scaled(d, s, sel);
+      }
+    }
+    return b;
+  }
   template <class A, int MCH>
   __device__ static void mma(const u32x4_t& w, const P& p, const u32x4_t (&xv)[MCH][4], f32x4_t (&yacc)[MCH]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t d = w[i];
-      u32x4_t b;
-      if (NV) {
-        // E4M3 scales carry mantissa bits: decode to fp32, scale, pack (e2m1 * s_b has <= 6
-        // significant bits, exact in bf16 / fp16, so taking the upper half is exact for bf16)
-        const float s = i < 2 ? p.s0 : p.s1;
-#pragma unroll
-        for (int sel = 0; sel < 4; ++sel) {
-          const f32x2_t f = A::fp4_pair_f32(d, sel);
-          b[sel] = A::pack_exact(f[0] * s, f[1] * s);
-        }
-      } else {
-#pragma unroll
-        for (int sel = 0; sel < 4; ++sel) b[sel] = A::fp4_pair_scaled(d, p.s0, sel);
-      }
+      const u32x4_t b = bfrag<A>(w, p, i);
 #pragma unroll
       for (int c = 0; c < MCH; ++c) yacc[c] = A::mfma(xv[c][i], b, yacc[c]);
     }
   }
+  // The row-tiled kernels' hooks (sqx_skinny.h)
+  static constexpr int NG = 1, MPG = STEPS, kLoads = 2;
+  static constexpr bool kPlainBlocks = true, kScaledFrag = true, kConstOffset = true;
+  template <class A>
+  __device__ static float const_offset() { return 0.0f; }
+  template <class A>
+  __device__ static float offset(const P&, int) { return 0.0f; }
+  __device__ static float scale(const P&, int) { return 1.0f; }
+  static const float* global_scale(const Args& a) { return NV ? a.s_global : nullptr; }
   __device__ static float out_scale(const Args& a, int) { return NV ? *a.s_global : 1.0f; }
 };
 
@@ -953,6 +965,83 @@ extern "C" int sqx_fp4_linear(const uint8_t* wt, const uint8_t* st, int fmt, con
   }
 #undef SQX_F4
   SQX_REQUIRE(e == hipSuccess, SQX_E_HIP, "sqx_fp4_linear: launch failed: %s", hipGetErrorString(e));
+  return SQX_OK;
+}
+
+// The library's launch shape for 2..64 rows (16-bit output), from a sweep of MXFP4 weights at 2..63 rows, rotating
+// copies (GEMV -> row-tiled, us): the int4 table but for these, where FP4's cheaper decode (no sums, no group
+// scale) moves the best shape, and the GEMV in place of int4's multi-row GEMV:
+//   1024..4095 tiles, m <= 8   4 tiles x 4 waves (8192 -> 28672 at m = 4 / 8: 33.8 / 43.7 -> 24.8 / 25.7; at 32 rows the
+//                              int4 shape, 109.2 -> 33.0)
+//   384..1023 tiles, K >= 8192 two splits of 4 x 8 to 8 rows, else LDS-staged 2 x 8 in four splits (28672 -> 8192 at
+//                              m = 4 / 32: 38.7 / 110.1 -> 26.7 / 33.7)
+//   640..1023 tiles, shorter K 4 x 8 to 8 rows, LDS-staged 1 x 8 at 17..32 (4096 -> 14336 at m = 4 / 32: 11.0 / 34.2 ->
+//                              9.2 / 13.3)
+static SkinnyShape fp4_default_shape(int64_t m, int64_t rows, int64_t cols, bool have_ws) {
+  const int64_t T = ceil_div(rows, 16), KB = ceil_div(cols, 128);
+  if (m >= 2 && T >= 1024 && T < 4096 && m <= 8) return SkinnyShape{0, 4, 4, 1, false};
+  if (m >= 2 && T >= 384 && T < 1024 && KB >= 64 && have_ws)
+    return m <= 8 ? SkinnyShape{0, 4, 8, 2, false} : SkinnyShape{1, 2, 8, 4, false};
+  if (m >= 2 && T >= 640 && T < 1024 && m <= 8) return SkinnyShape{0, 4, 8, 1, false};
+  if (T >= 640 && T < 1024 && m > 16 && m <= 32) return SkinnyShape{1, 1, 8, 1, false};
+  SkinnyShape sh = skinny_default_shape(m, rows, cols, 128, have_ws);
+  if (sh.variant == 2) sh = SkinnyShape{0, 2, 8, 1, true};
+  return sh;
+}
+
+extern "C" int64_t sqx_fp4_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits) {
+  if (m <= 0 || m > 64 || rows <= 0 || cols <= 0) return 0;
+  const SkinnyShape sh = fp4_default_shape(m, rows, cols, true);
+  const int S = splits > 0 ? splits : sh.gemv ? 1 : sh.S;
+  return skinny_workspace_bytes(m, rows, skinny_splits(ceil_div(cols, 128), S));
+}
+
+extern "C" int sqx_fp4_skinny(const uint8_t* wt, const uint8_t* st, int fmt, const float* s_global, const void* x,
+                              int act_dtype, void* y, const void* bias, int64_t m, int64_t rows, int64_t cols,
+                              int variant, int tiles, int waves, int splits, void* ws, int64_t ws_bytes,
+                              sqx_stream_t stream) {
+  const char* fn = "sqx_fp4_skinny";
+  SkinnyShape sh = fp4_default_shape(m, rows, cols, ws != nullptr);
+  const int64_t KB = ceil_div(cols, 128);
+  // the GEMV: the library's choice for the shape, or a weight beyond the 32-bit offsets of a workgroup's tiles
+  if ((variant < 0 && tiles <= 0 && waves <= 0 && splits <= 0 && sh.gemv) || 4 * KB * 1024 >= ((int64_t)1 << 31))
+    return sqx_fp4_linear(wt, st, fmt, s_global, x, act_dtype, y, act_dtype, bias, m, rows, cols, 0, stream);
+  if (variant >= 0 && (variant != sh.variant || sh.gemv))
+    sh = variant == 0 ? SkinnyShape{0, 2, 8, 1, false} : SkinnyShape{1, 2, 4, 1, false};
+  if (variant > 1) sh.variant = variant;  // refused below
+  if (tiles > 0) sh.R = tiles;
+  if (waves > 0) sh.waves = waves;
+  if (splits > 0) sh.S = splits;
+  SQX_REQUIRE(m >= 1 && m <= 64 && rows > 0 && cols > 0 && cols % 32 == 0, SQX_E_ARG,
+              "%s: bad shape m=%lld rows=%lld cols=%lld (1..64 rows, cols %% 32 == 0)", fn, (long long)m, (long long)rows,
+              (long long)cols);
+  SQX_REQUIRE(fmt == SQX_FP4_MX || fmt == SQX_FP4_NV, SQX_E_ARG, "%s: bad fmt %d", fn, fmt);
+  SQX_REQUIRE(act_dtype == SQX_DTYPE_BF16 || act_dtype == SQX_DTYPE_F16, SQX_E_ARG, "%s: activations must be BF16 or F16",
+              fn);
+  SQX_REQUIRE(rows < ((int64_t)1 << 31) && 64 * cols * 2 < ((int64_t)1 << 31), SQX_E_ARG,
+              "%s: shape too large for 32-bit buffer offsets", fn);
+  SQX_REQUIRE(wt && st && x && y && (fmt == SQX_FP4_MX || s_global), SQX_E_ARG, "%s: null pointer", fn);
+  SQX_REQUIRE(reinterpret_cast<uintptr_t>(wt) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, SQX_E_ARG,
+              "%s: wt and x must be 16-byte aligned", fn);
+  SQX_REQUIRE((sh.variant == 0 && (sh.R == 2 || sh.R == 4) && sh.waves >= 1 && sh.waves <= kSkinnyMaxWaves) ||
+                  (sh.variant == 1 && (sh.R == 1 || sh.R == 2 || sh.R == 4) && (sh.waves == 4 || sh.waves == 8)),
+              SQX_E_ARG, "%s: bad launch shape (variant %d, tiles %d, waves %d, splits %d)", fn, sh.variant, sh.R, sh.waves,
+              sh.S);
+  const int S = skinny_splits(KB, sh.S);
+  SQX_REQUIRE(S == 1 || (ws && ws_bytes >= skinny_workspace_bytes(m, rows, S)), SQX_E_SPACE,
+              "%s: %d splits need a workspace of %lld bytes", fn, S, (long long)skinny_workspace_bytes(m, rows, S));
+  auto* part = static_cast<float*>(ws);
+  const auto* xp = static_cast<const uint16_t*>(x);
+  const auto* b16 = static_cast<const uint16_t*>(bias);
+  auto* y16 = static_cast<uint16_t*>(y);
+  hipStream_t s = as_stream(stream);
+  hipError_t e;
+#define SQX_F4S(ACT, NV)                                                                                             \
+  e = skinny_launch<ACT, WFp4<NV>>(WFp4<NV>::Args{wt, st, s_global}, xp, y16, b16, m, rows, cols, sh, part, ws_bytes, s)
+  if (act_dtype == SQX_DTYPE_BF16) { if (fmt == SQX_FP4_NV) SQX_F4S(ActBF16, true); else SQX_F4S(ActBF16, false); }
+  else { if (fmt == SQX_FP4_NV) SQX_F4S(ActF16, true); else SQX_F4S(ActF16, false); }
+#undef SQX_F4S
+  SQX_REQUIRE(e == hipSuccess, SQX_E_HIP, "%s: launch failed: %s", fn, hipGetErrorString(e));
   return SQX_OK;
 }
 

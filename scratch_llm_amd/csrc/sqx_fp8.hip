@@ -220,10 +220,7 @@ struct WFp8 {
   __device__ static void load(const Ctx& c, int kb, u32x4_t& w, P&) { w = bload128<2>(c.wr, c.wvo, (uint32_t)kb * 1024u); }
   __device__ static int xk(int i, int jg) { return 16 * jg + 8 * i; }
   template <bool HI>
-  __device__ static uint32_t pair(uint32_t d) {  // bytes 0,1 (HI false) or 2,3 of d as a bf16 pair
-    const f32x2_t f = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(d), HI);
-    return ActBF16::pack_exact(f[0], f[1]);
-  }
+  __device__ static uint32_t pair(uint32_t d) { return ActBF16::fp8_pair<HI>(d); }  // bytes 0,1 or 2,3 of d
   template <class A, int MCH>
   __device__ static void mma(const u32x4_t& w, const P&, const u32x4_t (&xv)[MCH][STEPS], f32x4_t (&yacc)[MCH]) {
 #pragma unroll
@@ -381,25 +378,6 @@ static int64_t fp8_round256(int64_t b) { return (b + 255) / 256 * 256; }
 static int64_t fp8_vals_bytes(int64_t m, int64_t cols) { return fp8_round256(m * cols * 2); }
 static int64_t fp8_part_offset(int64_t m, int64_t cols) { return fp8_vals_bytes(m, cols) + fp8_round256(m * 4); }
 
-// The launch the library picks for m rows (bf16 output), from a measured sweep of the Llama-3-8B
-// shapes (4096 -> 1024 / 4096 / 6144 / 28672, 14336 -> 4096) at m = 2..64. R tiles of 16 weight rows
-// per workgroup share each activation fragment, `waves` waves split its k-blocks, S workgroups split
-// K; `gemv` marks shapes where the GEMV (one workgroup per tile) is faster:
-//   >= 1024 tiles          R = 2 (m <= 8) or 4, 4 waves, no split;
-//   384 .. 1023 tiles      the GEMV for m <= 4, else R = 2 with 8 waves;
-//   fewer, K >= 8192       the GEMV for m <= 4, else 8 waves and 4 splits, R = 2 (m <= 8) or 4;
-//   fewer, shorter K       the GEMV for m <= 16, else R = 2, 8 waves, 2 splits (4 below 256 tiles).
-static SkinnyShape fp8_default_shape(int64_t m, int64_t rows, int64_t cols) {
-  const int64_t T = ceil_div(rows, 16);
-  const int64_t KB = ceil_div(cols, WFp8::KBLK);
-  SkinnyShape sh{0, 2, 8, 1, true};
-  if (m < 2 || m > 64) return sh;
-  if (T >= 1024) return SkinnyShape{0, m <= 8 ? 2 : 4, 4, 1, false};
-  if (T >= 384) return SkinnyShape{0, 2, 8, 1, m <= 4};
-  if (KB >= 128) return SkinnyShape{0, m <= 8 ? 2 : 4, 8, 4, m <= 4};
-  return SkinnyShape{0, 2, 8, T >= 256 ? 2 : 4, m <= 16};
-}
-
 // Rows from which sqx_fp8_linear runs the dequant GEMM (the GEMV takes 64 rows per pass over the weight).
 static bool fp8_use_gemm(int64_t m, int64_t rows, int64_t cols) { return m > 64 && gemm8_fits(m, rows, cols); }
 
@@ -412,7 +390,7 @@ static int64_t fp8_ws_bytes(int64_t m, int64_t rows, int64_t cols, const SkinnyS
 extern "C" int64_t sqx_fp8_linear_workspace_bytes(int64_t m, int64_t rows, int64_t cols) {
   // the dequant GEMM's partials are optional: without room for them it makes one pass per output tile
   const int64_t part = fp8_use_gemm(m, rows, cols) ? fp8_gemm_workspace_bytes(m, rows, cols) : 0;
-  return fp8_ws_bytes(m, rows, cols, fp8_default_shape(m, rows, cols)) + part;
+  return fp8_ws_bytes(m, rows, cols, skinny64_default_shape(m, rows, cols)) + part;
 }
 
 extern "C" int64_t sqx_fp8_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits) {
@@ -474,7 +452,7 @@ static int fp8_linear_impl(const uint8_t* wt, const float* w_scale, const void* 
 extern "C" int sqx_fp8_linear(const uint8_t* wt, const float* w_scale, const void* x, int act_dtype, void* y, int y_dtype,
                               const void* bias, int64_t m, int64_t rows, int64_t cols, int k_slices, void* ws,
                               int64_t ws_bytes, sqx_stream_t stream) {
-  SkinnyShape sh = fp8_default_shape(m, rows, cols);
+  SkinnyShape sh = skinny64_default_shape(m, rows, cols);
   if (k_slices > 0 || y_dtype != SQX_DTYPE_BF16) sh.gemv = true;
   return fp8_linear_impl(wt, w_scale, x, act_dtype, y, y_dtype, bias, m, rows, cols, k_slices, sh, ws, ws_bytes, stream,
                          "sqx_fp8_linear");

@@ -9,7 +9,7 @@
 // Tiled int8 layout (the weight-only linear): block (t, kb) = 1 KiB covering 16 rows x 64 columns;
 // lane L owns the 16 codes of row 16t + (L & 15), columns kb*64 + 16(L >> 4) + e, stored as
 // u = q + 128 in byte e. Per-row fp32 scales are read in the epilogue.
-#include "sqx_gemv.h"
+#include "sqx_skinny.h"
 
 namespace sqx {
 
@@ -310,6 +310,26 @@ struct WInt8 {
     y0 += fmaf(-128.0f, sig[0], acc[0]);
   }
   __device__ static float out_scale(const Args& a, int n) { return a.scale[n]; }
+
+  // The row-tiled kernels' hooks (sqx_skinny.h): the codes as their signed values, exact in bf16 and fp16, so a
+  // block's MFMAs chain straight into the output sums.
+  static constexpr int MPG = STEPS;
+  static constexpr bool kPlainBlocks = true, kConstOffset = true;
+  __device__ static Ctx ctx_tiles(const Args& a, int t, int nt, int KB, int lane) {
+    return Ctx{make_rsrc(a.wt + (int64_t)t * KB * 1024, (uint32_t)nt * (uint32_t)KB * 1024u), (uint32_t)lane * 16u};
+  }
+  template <class A>
+  __device__ static u32x4_t bfrag(const u32x4_t& w, int i) {
+    const uint32_t d0 = w[2 * i] ^ 0x80808080u, d1 = w[2 * i + 1] ^ 0x80808080u;  // q + 128 -> two's complement
+    return u32x4_t{A::pack_exact(sbyte_f32<0>(d0), sbyte_f32<1>(d0)), A::pack_exact(sbyte_f32<2>(d0), sbyte_f32<3>(d0)),
+                   A::pack_exact(sbyte_f32<0>(d1), sbyte_f32<1>(d1)), A::pack_exact(sbyte_f32<2>(d1), sbyte_f32<3>(d1))};
+  }
+  template <class A>
+  __device__ static float const_offset() { return 0.0f; }
+  template <class A>
+  __device__ static float offset(const P&, int) { return 0.0f; }
+  __device__ static float scale(const P&, int) { return 1.0f; }
+  static const float* out_scales(const Args& a) { return a.scale; }
 };
 
 // One thread per output dword of the tiled int8 weight.
@@ -548,5 +568,53 @@ extern "C" int sqx_int8_linear(const uint8_t* wt, const float* scale, const void
                                                 static_cast<const uint16_t*>(bias), nullptr, m, rows, cols, k_slices,
                                                 as_stream(stream));
   SQX_REQUIRE(e == hipSuccess, SQX_E_HIP, "sqx_int8_linear: launch failed: %s", hipGetErrorString(e));
+  return SQX_OK;
+}
+
+extern "C" int64_t sqx_int8_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits) {
+  if (m <= 0 || m > 64 || rows <= 0 || cols <= 0) return 0;
+  const SkinnyShape sh = skinny64_default_shape(m, rows, cols);
+  const int S = splits > 0 ? splits : sh.gemv ? 1 : sh.S;
+  return skinny_workspace_bytes(m, rows, skinny_splits(ceil_div(cols, 64), S));
+}
+
+extern "C" int sqx_int8_skinny(const uint8_t* wt, const float* scale, const void* x, int act_dtype, void* y,
+                               const void* bias, int64_t m, int64_t rows, int64_t cols, int tiles, int waves,
+                               int splits, void* ws, int64_t ws_bytes, sqx_stream_t stream) {
+  const char* fn = "sqx_int8_skinny";
+  const bool choose = tiles <= 0 && waves <= 0 && splits <= 0;
+  SkinnyShape sh = skinny64_default_shape(m, rows, cols);
+  const int64_t KB = ceil_div(cols, 64);
+  // the GEMV: the library's choice for the shape, or a row tile group beyond the 32-bit offsets
+  if ((choose && sh.gemv) || 4 * KB * 1024 >= ((int64_t)1 << 31))
+    return sqx_int8_linear(wt, scale, x, act_dtype, y, bias, m, rows, cols, 0, stream);
+  if (!choose) sh = SkinnyShape{0, tiles > 0 ? tiles : 2, waves > 0 ? waves : 8, splits > 0 ? splits : 1, false};
+  SQX_REQUIRE(m >= 1 && m <= 64 && rows > 0 && cols > 0 && cols % 8 == 0, SQX_E_ARG,
+              "%s: bad shape m=%lld rows=%lld cols=%lld (1..64 rows, cols %% 8 == 0)", fn, (long long)m, (long long)rows,
+              (long long)cols);
+  SQX_REQUIRE(act_dtype == SQX_DTYPE_BF16 || act_dtype == SQX_DTYPE_F16, SQX_E_ARG, "%s: activations must be BF16 or F16",
+              fn);
+  SQX_REQUIRE(rows < ((int64_t)1 << 31) && 64 * cols * 2 < ((int64_t)1 << 31), SQX_E_ARG,
+              "%s: shape too large for 32-bit buffer offsets", fn);
+  SQX_REQUIRE(wt && scale && x && y, SQX_E_ARG, "%s: null pointer", fn);
+  SQX_REQUIRE(reinterpret_cast<uintptr_t>(wt) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, SQX_E_ARG,
+              "%s: wt and x must be 16-byte aligned", fn);
+  SQX_REQUIRE((sh.R == 2 || sh.R == 4) && sh.waves >= 1 && sh.waves <= kSkinnyMaxWaves, SQX_E_ARG,
+              "%s: bad launch shape (tiles %d, waves %d, splits %d)", fn, sh.R, sh.waves, sh.S);
+  const int S = skinny_splits(KB, sh.S);
+  if (choose && S > 1 && (ws == nullptr || ws_bytes < skinny_workspace_bytes(m, rows, S))) sh.S = 1;
+  else
+    SQX_REQUIRE(S == 1 || (ws && ws_bytes >= skinny_workspace_bytes(m, rows, S)), SQX_E_SPACE,
+                "%s: %d splits need a workspace of %lld bytes", fn, S, (long long)skinny_workspace_bytes(m, rows, S));
+  const WInt8::Args a{wt, scale};
+  const auto* xp = static_cast<const uint16_t*>(x);
+  const auto* b16 = static_cast<const uint16_t*>(bias);
+  auto* y16 = static_cast<uint16_t*>(y);
+  auto* part = static_cast<float*>(ws);
+  const hipError_t e =
+      act_dtype == SQX_DTYPE_BF16
+          ? skinny_launch<ActBF16, WInt8>(a, xp, y16, b16, m, rows, cols, sh, part, ws_bytes, as_stream(stream))
+          : skinny_launch<ActF16, WInt8>(a, xp, y16, b16, m, rows, cols, sh, part, ws_bytes, as_stream(stream));
+  SQX_REQUIRE(e == hipSuccess, SQX_E_HIP, "%s: launch failed: %s", fn, hipGetErrorString(e));
   return SQX_OK;
 }

@@ -29,7 +29,8 @@
 //   W::offset<A>(p, g)                     magic + zero point of group g (lane's weight row)
 //   W::scale(p, g)                         group scale (lane's weight row)
 // A policy whose codes decode to the weight values themselves (no offset, no group scale) declares
-// kPlainBlocks = true instead: its MFMAs chain straight into the output sums. A per-token factor
+// kPlainBlocks = true instead: its MFMAs chain straight into the output sums (FP4's block scale is a power of
+// two or a short E4M3 factor, exact in the decoded fragment: kScaledFrag, bfrag<A>(w, p, i)). A per-token factor
 // (kRowScale, row_scale) is applied in the epilogue as in the GEMV, and with K splits by the reduce,
 // which takes the factors from W::row_scales(args) [m] and W::out_scales(args) [n].
 #pragma once
@@ -44,6 +45,16 @@ template <class W, class = void>
 struct plain_blocks : std::false_type {};
 template <class W>
 struct plain_blocks<W, std::void_t<decltype(W::kPlainBlocks)>> : std::integral_constant<bool, W::kPlainBlocks> {};
+// A policy whose decoded fragment takes the block's scale in (kScaledFrag) gets its parameters.
+template <class W, class = void>
+struct scaled_frag : std::false_type {};
+template <class W>
+struct scaled_frag<W, std::void_t<decltype(W::kScaledFrag)>> : std::integral_constant<bool, W::kScaledFrag> {};
+template <class A, class W>
+__device__ __forceinline__ u32x4_t w_bfrag(const u32x4_t& w, const typename W::P& p, int i) {
+  if constexpr (scaled_frag<W>::value) return W::template bfrag<A>(w, p, i);
+  else return W::template bfrag<A>(w, i);
+}
 // KiB of weights in flight per compute wave of the LDS-staged variant (a ring of this many k-blocks
 // over the wave's R tiles)
 #ifndef SQX_SKINNY_RING_KIB
@@ -202,7 +213,7 @@ __global__ __launch_bounds__((64 * skinny_max_waves(MCH, R, W::NG, W::kConstOffs
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int i = 0; i < STEPS; ++i) b[r][i] = W::template bfrag<A>(w[r], i);
+      for (int i = 0; i < STEPS; ++i) b[r][i] = w_bfrag<A, W>(w[r], p[r], i);
       pc[r] = p[r];
     }
     u32x4_t xn[MCH][STEPS];
@@ -413,7 +424,7 @@ __global__ __launch_bounds__(256 * KG) void skinny_lds_kernel(const typename W::
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int i = 0; i < STEPS; ++i) bcur[r][i] = W::template bfrag<A>(wring[0][r], i);
+      for (int i = 0; i < STEPS; ++i) bcur[r][i] = w_bfrag<A, W>(wring[0][r], pring[0][r], i);
       pcur[r] = pring[0][r];
     }
   }
@@ -432,7 +443,7 @@ __global__ __launch_bounds__(256 * KG) void skinny_lds_kernel(const typename W::
 #pragma unroll
         for (int r = 0; r < R; ++r) {
 #pragma unroll
-          for (int i = 0; i < STEPS; ++i) bcur[r][i] = W::template bfrag<A>(wring[d][r], i);
+          for (int i = 0; i < STEPS; ++i) bcur[r][i] = w_bfrag<A, W>(wring[d][r], pring[d][r], i);
           pcur[r] = pring[d][r];
         }
       }
@@ -456,47 +467,59 @@ __global__ __launch_bounds__(256 * KG) void skinny_lds_kernel(const typename W::
       } else {
         u32x4_t bnext[R][STEPS];
         typename W::P pnext[R];
-        f32x4_t xs[MCH];
+        constexpr bool PLAIN = plain_blocks<W>::value;
+        f32x4_t acc[PLAIN ? 1 : R][MCH];
+        if constexpr (PLAIN) {
 #pragma unroll
-        for (int c = 0; c < MCH; ++c) xs[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          for (int i = 0; i < STEPS; ++i)
 #pragma unroll
-        for (int i = 0; i < STEPS; ++i)
+            for (int r = 0; r < R; ++r)
 #pragma unroll
-          for (int c = 0; c < MCH; ++c) xs[c] = A::mfma(xv[c][i], sumv, xs[c]);
-        f32x4_t acc[R][MCH];
+              for (int c = 0; c < MCH; ++c) yacc[r][c] = A::mfma(xv[c][i], bcur[r][i], yacc[r][c]);
+        } else {
+          f32x4_t xs[MCH];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          if constexpr (W::kConstOffset) {
+          for (int c = 0; c < MCH; ++c) xs[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int c = 0; c < MCH; ++c) acc[r][c] = xs[c];
-          } else {
-            const float o = -W::template offset<A>(pcur[r], 0);
+          for (int i = 0; i < STEPS; ++i)
 #pragma unroll
-            for (int c = 0; c < MCH; ++c)
+            for (int c = 0; c < MCH; ++c) xs[c] = A::mfma(xv[c][i], sumv, xs[c]);
 #pragma unroll
-              for (int j = 0; j < 4; ++j) acc[r][c][j] = o * xs[c][j];
+          for (int r = 0; r < R; ++r) {
+            if constexpr (W::kConstOffset) {
+#pragma unroll
+              for (int c = 0; c < MCH; ++c) acc[r][c] = xs[c];
+            } else {
+              const float o = -W::template offset<A>(pcur[r], 0);
+#pragma unroll
+              for (int c = 0; c < MCH; ++c)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[r][c][j] = o * xs[c][j];
+            }
           }
+#pragma unroll
+          for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+              for (int c = 0; c < MCH; ++c) acc[r][c] = A::mfma(xv[c][i], bcur[r][i], acc[r][c]);
         }
-#pragma unroll
-        for (int i = 0; i < STEPS; ++i)
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int c = 0; c < MCH; ++c) acc[r][c] = A::mfma(xv[c][i], bcur[r][i], acc[r][c]);
         // decode step s+1 while the chains run (after the last step the result goes unused)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
 #pragma unroll
-          for (int i = 0; i < STEPS; ++i) bnext[r][i] = W::template bfrag<A>(wring[dn][r], i);
+          for (int i = 0; i < STEPS; ++i) bnext[r][i] = w_bfrag<A, W>(wring[dn][r], pring[dn][r], i);
           pnext[r] = pring[dn][r];
         }
+        if constexpr (!PLAIN) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const float sc = W::scale(pcur[r], 0);
+          for (int r = 0; r < R; ++r) {
+            const float sc = W::scale(pcur[r], 0);
 #pragma unroll
-          for (int c = 0; c < MCH; ++c)
+            for (int c = 0; c < MCH; ++c)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) yacc[r][c][j] = fmaf(sc, acc[r][c][j], yacc[r][c][j]);
+              for (int j = 0; j < 4; ++j) yacc[r][c][j] = fmaf(sc, acc[r][c][j], yacc[r][c][j]);
+          }
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -578,13 +601,14 @@ __global__ __launch_bounds__(256 * KG) void skinny_lds_kernel(const typename W::
   }
 }
 
-// y[m, n] = act(sum over s in order of part[s][m][n] (* rs[m] * cs[n] when rs is given) + bias[n]);
+// y[m, n] = act(sum over s in order of part[s][m][n] (* rs[m] when given) (* cs[n]) (* *gs) + bias[n]);
 // four outputs per thread.
 template <class A>
 __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restrict__ part, int S, int M, int N,
                                                             const uint16_t* __restrict__ bias,
                                                             uint16_t* __restrict__ y, const float* __restrict__ rs,
-                                                            const float* __restrict__ cs) {
+                                                            const float* __restrict__ cs,
+                                                            const float* __restrict__ gs) {
   const int64_t total = (int64_t)M * N;
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= total) return;
@@ -598,10 +622,12 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
       for (int j = 0; j < 4; ++j) v[j] += q[j];
     }
     const int n = static_cast<int>(i % N);
-    if (rs) {
-      const float r = rs[i / N];
+    const float r = rs ? rs[i / N] : 1.0f, g = gs ? *gs : 1.0f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = v[j] * r * cs[n + j];
+    for (int j = 0; j < 4; ++j) {
+      if (rs) v[j] *= r;
+      if (cs) v[j] *= cs[n + j];
+      if (gs) v[j] *= g;
     }
     uint32_t lo, hi;
     float o[4];
@@ -614,7 +640,9 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
     for (int64_t e = i; e < i + 4 && e < total; ++e) {
       float v = part[e];
       for (int s = 1; s < S; ++s) v += part[(int64_t)s * total + e];
-      if (rs) v = v * rs[e / N] * cs[e % N];
+      if (rs) v *= rs[e / N];
+      if (cs) v *= cs[e % N];
+      if (gs) v *= *gs;
       if (bias) v += A::to_f32(bias[e % N]);
       y[e] = A::from_f32(v);
     }
@@ -709,6 +737,25 @@ inline SkinnyShape skinny_default_shape(int64_t m, int64_t rows, int64_t cols, i
   return s;
 }
 
+// The launch the library picks for m rows of the formats with 64-column blocks (FP8, int8; 16-bit output), from
+// a measured sweep of FP8 at the Llama-3-8B shapes (4096 -> 1024 / 4096 / 6144 / 28672, 14336 -> 4096) at m = 2..64. R tiles of 16 weight rows
+// per workgroup share each activation fragment, `waves` waves split its k-blocks, S workgroups split
+// K; `gemv` marks shapes where the GEMV (one workgroup per tile) is faster:
+//   >= 1024 tiles          R = 2 (m <= 8) or 4, 4 waves, no split;
+//   384 .. 1023 tiles      the GEMV for m <= 4, else R = 2 with 8 waves;
+//   fewer, K >= 8192       the GEMV for m <= 4, else 8 waves and 4 splits, R = 2 (m <= 8) or 4;
+//   fewer, shorter K       the GEMV for m <= 16, else R = 2, 8 waves, 2 splits (4 below 256 tiles).
+inline SkinnyShape skinny64_default_shape(int64_t m, int64_t rows, int64_t cols) {
+  const int64_t T = ceil_div(rows, 16);
+  const int64_t KB = ceil_div(cols, 64);
+  SkinnyShape sh{0, 2, 8, 1, true};
+  if (m < 2 || m > 64) return sh;
+  if (T >= 1024) return SkinnyShape{0, m <= 8 ? 2 : 4, 4, 1, false};
+  if (T >= 384) return SkinnyShape{0, 2, 8, 1, m <= 4};
+  if (KB >= 128) return SkinnyShape{0, m <= 8 ? 2 : 4, 8, 4, m <= 4};
+  return SkinnyShape{0, 2, 8, T >= 256 ? 2 : 4, m <= 16};
+}
+
 inline int64_t skinny_workspace_bytes(int64_t m, int64_t rows, int S) { return S > 1 ? (int64_t)S * m * rows * 4 : 0; }
 
 // The number of K splits a launch actually makes for S requested over KB k-blocks (no empty split).
@@ -716,6 +763,21 @@ inline int skinny_splits(int64_t KB, int S) {
   if (S < 1) S = 1;
   if (S > KB) S = static_cast<int>(KB);
   return static_cast<int>(ceil_div(KB, ceil_div(KB, S)));
+}
+
+// The factors the split reduce applies for a policy: out_scales(args) [n], global_scale(args) (one value).
+template <class W, class = void>
+struct has_out_scales : std::false_type {};
+template <class W>
+struct has_out_scales<W, std::void_t<decltype(&W::out_scales)>> : std::true_type {};
+template <class W, class = void>
+struct has_global_scale : std::false_type {};
+template <class W>
+struct has_global_scale<W, std::void_t<decltype(&W::global_scale)>> : std::true_type {};
+template <class W>
+const float* global_scale(const typename W::Args& wa) {
+  if constexpr (has_global_scale<W>::value) return W::global_scale(wa);
+  else return nullptr;
 }
 
 // The LDS-staged variant: R (1, 2 or 4) tiles per wave, 4 waves per workgroup, S splits along K.
@@ -778,7 +840,7 @@ hipError_t skinny_lds_launch(const typename W::Args& wa, const uint16_t* x, uint
   if (e != hipSuccess || !split || !reduce) return e;
   const int64_t quads = ceil_div(m * rows, 4);
   hipLaunchKernelGGL(skinny_reduce_kernel<A>, dim3(static_cast<unsigned>(ceil_div(quads, 256))), dim3(256), 0, stream,
-                     ws, S, M, N, bias, y, nullptr, nullptr);
+                     ws, S, M, N, bias, y, nullptr, nullptr, global_scale<W>(wa));
   return hipGetLastError();
 }
 
@@ -841,12 +903,10 @@ hipError_t skinny_launch(const typename W::Args& wa, const uint16_t* x, uint16_t
   const int64_t quads = ceil_div(m * rows, 4);
   const float* rs = nullptr;
   const float* cs = nullptr;
-  if constexpr (has_row_scale<W>::value) {
-    rs = W::row_scales(wa);
-    cs = W::out_scales(wa);
-  }
+  if constexpr (has_row_scale<W>::value) rs = W::row_scales(wa);
+  if constexpr (has_out_scales<W>::value) cs = W::out_scales(wa);
   hipLaunchKernelGGL(skinny_reduce_kernel<A>, dim3(static_cast<unsigned>(ceil_div(quads, 256))), dim3(256), 0, stream,
-                     ws, S, M, N, bias, y, rs, cs);
+                     ws, S, M, N, bias, y, rs, cs, global_scale<W>(wa));
   return hipGetLastError();
 }
 

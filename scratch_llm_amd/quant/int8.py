@@ -267,15 +267,14 @@ def untile_int8(tw: Int8Tiled) -> Tensor:
     return q
 
 
-# Activation rows from which the tiled int8 linear runs the prefill GEMM (the streaming kernel makes one
-# pass over the weight per 64 rows).
+# Activation rows from which the tiled int8 linear runs the prefill GEMM.
 GEMM_MIN_M = 65
 
 
 def int8_linear_tiled(x: Tensor, tw: Int8Tiled, bias: Tensor | None = None, k_slices: int | None = None) -> Tensor:
-    """``x @ (q * s).T (+ bias)`` for a tiled int8 weight; ``x`` bf16 / fp16 ``[..., in]``. Up to
-    ``GEMM_MIN_M - 1`` rows, or with ``k_slices`` set, on the streaming decode kernel; from there on the
-    prefill GEMM."""
+    """``x @ (q * s).T (+ bias)`` for a tiled int8 weight; ``x`` bf16 / fp16 ``[..., in]``. One row,
+    or any with ``k_slices`` set, on the streaming decode GEMV; 2..``GEMM_MIN_M - 1`` rows on the library's
+    choice of the GEMV and the row-tiled kernel; from there on the prefill GEMM."""
     *batch, k = x.shape
     if k != tw.cols:
         raise ValueError(f"x has in_features={k}, weight expects {tw.cols}")
@@ -296,6 +295,13 @@ def int8_linear_tiled(x: Tensor, tw: Int8Tiled, bias: Tensor | None = None, k_sl
             _lib.check(lib.sqx_int8_gemm(tw.wt.data_ptr(), tw.scale.data_ptr(), x2.data_ptr(), _lib.sqx_dtype(x.dtype),
                                          y.data_ptr(), _lib.ptr(b), m, tw.rows, k, *_lib.ws_args(ws),
                                          _lib.stream_ptr(dev)), "int8_linear")
+            return y.reshape(*batch, tw.rows)
+        if 2 <= m < GEMM_MIN_M and k_slices is None:
+            nb = int(lib.sqx_int8_skinny_workspace_bytes(m, tw.rows, k, 0))
+            ws = torch.empty(nb // 4, dtype=torch.float32, device=dev) if nb > 0 else None
+            _lib.check(lib.sqx_int8_skinny(tw.wt.data_ptr(), tw.scale.data_ptr(), x2.data_ptr(), _lib.sqx_dtype(x.dtype),
+                                           y.data_ptr(), _lib.ptr(b), m, tw.rows, k, 0, 0, 0, *_lib.ws_args(ws),
+                                           _lib.stream_ptr(dev)), "int8_linear")
             return y.reshape(*batch, tw.rows)
         _lib.check(lib.sqx_int8_linear(tw.wt.data_ptr(), tw.scale.data_ptr(), x2.data_ptr(),
                                        _lib.sqx_dtype(x.dtype), y.data_ptr(), _lib.ptr(b), m, tw.rows, tw.cols,

@@ -377,6 +377,12 @@ def fp4_linear_tiled(x: Tensor, tw: FP4Tiled, bias: Tensor | None = None, out_dt
             _lib.check(lib.sqx_fp4_gemm(tw.wt.data_ptr(), tw.st.data_ptr(), tw.fmt, _lib.ptr(tw.s_global), x2.data_ptr(),
                                         _lib.sqx_dtype(x.dtype), y.data_ptr(), ydt, _lib.ptr(b), m, tw.rows, tw.cols,
                                         *_lib.ws_args(ws), s), "fp4_linear")
+        elif 2 <= m < GEMM_MIN_M and k_slices is None and not yf32:
+            nb = int(lib.sqx_fp4_skinny_workspace_bytes(m, tw.rows, tw.cols, 0))
+            ws = torch.empty(nb // 4, dtype=torch.float32, device=dev) if nb > 0 else None
+            _lib.check(lib.sqx_fp4_skinny(tw.wt.data_ptr(), tw.st.data_ptr(), tw.fmt, _lib.ptr(tw.s_global), x2.data_ptr(),
+                                          _lib.sqx_dtype(x.dtype), y.data_ptr(), _lib.ptr(b), m, tw.rows, tw.cols, -1, 0,
+                                          0, 0, *_lib.ws_args(ws), s), "fp4_linear")
         else:
             _lib.check(lib.sqx_fp4_linear(tw.wt.data_ptr(), tw.st.data_ptr(), tw.fmt, _lib.ptr(tw.s_global),
                                           x2.data_ptr(), _lib.sqx_dtype(x.dtype), y.data_ptr(), ydt, _lib.ptr(b), m,
