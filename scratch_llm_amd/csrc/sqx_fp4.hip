@@ -9,8 +9,9 @@
 // reference's row-major packed weight. Scales per block (t, kb): MXFP4 64 bytes, byte L the E8M0
 // scale of lane L's 32 columns; NVFP4 128 bytes, bytes 2L and 2L+1 the E4M3 scales of lane L's two
 // 16-column halves. Padding rows / columns hold code 0 and scale byte 0.
-#include "sqx_skinny.h"
 #include "sqx_mx.h"
+#include "sqx_quant.h"
+#include "sqx_skinny.h"
 
 #include <float.h>
 
@@ -136,6 +137,53 @@ __global__ __launch_bounds__(256) void fp4_quantize_kernel(const void* __restric
   }
 }
 
+// The same for blocks of LPB * 8 elements (a power of two) that all lie below n, and aligned pointers: LPB lanes a
+// block, 8 consecutive elements each, the block maximum joined with shuffles, the division shared by the block.
+// 14336 x 4096 in bf16, mx / nv: 525 / 383 -> 48 / 110 us (one thread walked a block before).
+template <bool NV, int LPB>
+__global__ __launch_bounds__(256) void fp4_quantize8_kernel(const void* __restrict__ x, int dtype, int64_t n8,
+                                                            uint8_t* __restrict__ codes, float* __restrict__ s_block,
+                                                            uint8_t* __restrict__ e8m0,
+                                                            const float* __restrict__ s_global) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool live = i < n8;  // the lanes of a block are live or not together
+  float v[8];
+  load8_f32(x, dtype, live ? 8 * i : 0, v);
+  float amax = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) amax = amax_step(amax, v[e]);
+#pragma unroll
+  for (int o = 1; o < LPB; o <<= 1) amax = amax_step(amax, __shfl_xor(amax, o, 64));
+  if (!live) return;
+  const bool lead = (threadIdx.x & (LPB - 1)) == 0;
+  uint32_t w[2] = {0u, 0u};
+  if (NV) {
+    const float sg = *s_global;
+    const float sb = quantize_e4m3(__fdiv_rn(__fdiv_rn(amax, 6.0f), sg));
+    float scale = sg * sb;
+    if (scale < kTiny) scale = kTiny;
+    if (lead) s_block[i / LPB] = sb;
+    const SharedDiv sd = shared_div(scale);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float t = div_by(sd, v[e]);
+      // a code's sign bit says that the quotient is below zero: one that the shared division flushed to zero
+      // is divided again (a true zero has no sign bit either way)
+      if (t == 0.0f && v[e] != 0.0f) t = __fdiv_rn(v[e], scale);
+      w[e >> 2] |= e2m1_code(t) << (8 * (e & 3));
+    }
+  } else {
+    const int ex = mx_exponent(amax);
+    const float scale = ex == 128 ? __builtin_nanf("") : ldexpf(1.0f, ex);
+    if (lead) s_block[i / LPB] = scale;
+    if (lead && e8m0) e8m0[i / LPB] = static_cast<uint8_t>(ex == 128 ? 255 : ex + 127);
+    const float inv = ex == 128 ? __builtin_nanf("") : ldexpf(1.0f, -ex);  // v * 2**-e rounds as v / 2**e does
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e >> 2] |= e2m1_code(v[e] * inv) << (8 * (e & 3));
+  }
+  *reinterpret_cast<u32x2v_t*>(codes + 8 * i) = u32x2v_t{w[0], w[1]};
+}
+
 // mxfp4_quantize of the rows of x [m, k] (k % 32 == 0, so each of the reference's flattened
 // 32-blocks lies in one row) written straight into the tiled layout: one thread per 16-byte lane
 // chunk q of the padded [16 * ceil(m/16), 128 * KB] grid, i.e. row 16t + (L & 15), columns
@@ -242,9 +290,18 @@ __global__ __launch_bounds__(256) void mxfp4_fake_quant_rows_kernel(const void* 
 static constexpr int kAmaxParts = 512;
 
 __global__ __launch_bounds__(256) void amax_partial_kernel(const void* __restrict__ x, int dtype, int64_t n,
-                                                           float* __restrict__ part) {
+                                                           float* __restrict__ part, int vec) {
   __shared__ float red[256];
   float m = 0.0f;
+  if (vec) {  // n % 8 == 0, aligned
+#pragma unroll 4
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n / 8; i += (int64_t)gridDim.x * blockDim.x) {
+      float v[8];
+      load8_f32(x, dtype, 8 * i, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m = amax_step(m, v[e]);
+    }
+  } else
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     m = amax_step(m, load_as_f32(x, dtype, i));
   red[threadIdx.x] = m;
@@ -295,17 +352,34 @@ __global__ __launch_bounds__(256) void fp4_dequantize_kernel(const uint8_t* __re
 template <bool PACKED>
 __global__ __launch_bounds__(256) void fp4_tile_weights_kernel(const uint8_t* __restrict__ src, int64_t rows,
                                                                int64_t cols, int64_t KB, int64_t n_chunks,
-                                                               u32x4_t* __restrict__ wt) {
+                                                               u32x4_t* __restrict__ wt, int vec) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= n_chunks) return;
   const int L = static_cast<int>(q & 63);
-  const int64_t blk = q >> 6;
-  const int64_t t = blk / KB;
+  const uint32_t blk = static_cast<uint32_t>(q >> 6);  // blocks of 1 KiB: below 2**32
+  const int64_t t = blk / static_cast<uint32_t>(KB);
   const int64_t kb = blk - t * KB;
   const int64_t r = 16 * t + (L & 15);
   const int64_t c0 = kb * 128 + 32 * (L >> 4);
   uint32_t d[4] = {0u, 0u, 0u, 0u};
-  if (r < rows) {
+  if (vec && r < rows && c0 + 32 <= cols) {
+    // the lane's 32 codes are whole and 16-byte aligned in the source (14336 x 4096 codes: 129 -> 23 us)
+    const u32x4_t* p = reinterpret_cast<const u32x4_t*>(src + (PACKED ? (r * cols + c0) / 2 : r * cols + c0));
+    if (PACKED) {
+      wt[q] = p[0];
+      return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const u32x4_t v = p[h];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {  // four codes, one per byte -> four nibbles
+        uint32_t b = v[j] & 0x0F0F0F0Fu;
+        b = (b | (b >> 4)) & 0x00FF00FFu;
+        d[2 * h + (j >> 1)] |= ((b | (b >> 8)) & 0xFFFFu) << (16 * (j & 1));
+      }
+    }
+  } else if (r < rows) {
 #pragma unroll 4
     for (int e = 0; e < 32; ++e) {
       const int64_t c = c0 + e;
@@ -714,6 +788,23 @@ extern "C" int sqx_quantize_e8m0(const float* v, int64_t n, float* out, sqx_stre
   return SQX_OK;
 }
 
+// Blocks of 16, 32, 64 or 128 elements, all whole, with 16-byte loads and 8-byte stores.
+static bool quantize8_fits(const void* x, int64_t n, int64_t block, const uint8_t* codes) {
+  return (block == 16 || block == 32 || block == 64 || block == 128) && n % block == 0 &&
+         reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(codes) % 8 == 0;
+}
+template <bool NV>
+static void launch_quantize8(const void* x, int dtype, int64_t n, int64_t block, uint8_t* codes, float* s_block,
+                             uint8_t* e8m0, const float* s_global, hipStream_t s) {
+#define SQX_QB(L)                                                                                                    \
+  case 8 * L:                                                                                                        \
+    hipLaunchKernelGGL((fp4_quantize8_kernel<NV, L>), grid_for(n / 8), dim3(256), 0, s, x, dtype, n / 8, codes, s_block, \
+                       e8m0, s_global);                                                                              \
+    break
+  switch (block) { SQX_QB(2); SQX_QB(4); SQX_QB(8); SQX_QB(16); }
+#undef SQX_QB
+}
+
 extern "C" int sqx_mxfp4_quantize(const void* x, int dtype, int64_t n, int64_t block, uint8_t* codes,
                                   float* s_block, uint8_t* e8m0, sqx_stream_t stream) {
   SQX_REQUIRE(n >= 0 && block >= 1 && block <= 4096 && is_float_dtype(dtype), SQX_E_ARG,
@@ -721,8 +812,11 @@ extern "C" int sqx_mxfp4_quantize(const void* x, int dtype, int64_t n, int64_t b
   if (n == 0) return SQX_OK;
   SQX_REQUIRE(x && codes && s_block, SQX_E_ARG, "sqx_mxfp4_quantize: null pointer");
   const int64_t nb = ceil_div(n, block);
-  hipLaunchKernelGGL(fp4_quantize_kernel<false>, grid_for(nb), dim3(256), 0, as_stream(stream), x, dtype, n, nb,
-                     static_cast<int>(block), codes, s_block, e8m0, nullptr);
+  if (quantize8_fits(x, n, block, codes))
+    launch_quantize8<false>(x, dtype, n, block, codes, s_block, e8m0, nullptr, as_stream(stream));
+  else
+    hipLaunchKernelGGL(fp4_quantize_kernel<false>, grid_for(nb), dim3(256), 0, as_stream(stream), x, dtype, n, nb,
+                       static_cast<int>(block), codes, s_block, e8m0, nullptr);
   SQX_LAUNCH_CHECK("sqx_mxfp4_quantize");
   return SQX_OK;
 }
@@ -751,13 +845,17 @@ extern "C" int sqx_nvfp4_quantize(const void* x, int dtype, int64_t n, int64_t b
   const int parts = n == 0 ? 1 : static_cast<int>(std::min<int64_t>(kAmaxParts, ceil_div(n, 256)));
   if (n > 0) {
     SQX_REQUIRE(x && codes && s_block, SQX_E_ARG, "sqx_nvfp4_quantize: null pointer");
-    hipLaunchKernelGGL(amax_partial_kernel, dim3(parts), dim3(256), 0, s, x, dtype, n, part);
+    hipLaunchKernelGGL(amax_partial_kernel, dim3(parts), dim3(256), 0, s, x, dtype, n, part,
+                       n % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0);
   }
   hipLaunchKernelGGL(nv_global_scale_kernel, dim3(1), dim3(256), 0, s, part, n > 0 ? parts : 0, s_global);
   if (n > 0) {
     const int64_t nb = ceil_div(n, block);
-    hipLaunchKernelGGL(fp4_quantize_kernel<true>, grid_for(nb), dim3(256), 0, s, x, dtype, n, nb,
-                       static_cast<int>(block), codes, s_block, nullptr, s_global);
+    if (quantize8_fits(x, n, block, codes))
+      launch_quantize8<true>(x, dtype, n, block, codes, s_block, nullptr, s_global, s);
+    else
+      hipLaunchKernelGGL(fp4_quantize_kernel<true>, grid_for(nb), dim3(256), 0, s, x, dtype, n, nb,
+                         static_cast<int>(block), codes, s_block, nullptr, s_global);
   }
   SQX_LAUNCH_CHECK("sqx_nvfp4_quantize");
   return SQX_OK;
@@ -801,10 +899,13 @@ extern "C" int sqx_fp4_tile(const uint8_t* codes, int codes_packed, const void* 
   const int64_t KB = ceil_div(cols, 128);
   const int64_t chunks = ceil_div(rows, 16) * KB * 64;
   u32x4_t* w4 = reinterpret_cast<u32x4_t*>(wt);
+  const int vec = cols % 32 == 0 && reinterpret_cast<uintptr_t>(codes) % 16 == 0;
   if (codes_packed)
-    hipLaunchKernelGGL(fp4_tile_weights_kernel<true>, grid_for(chunks), dim3(256), 0, s, codes, rows, cols, KB, chunks, w4);
+    hipLaunchKernelGGL(fp4_tile_weights_kernel<true>, grid_for(chunks), dim3(256), 0, s, codes, rows, cols, KB, chunks,
+                       w4, vec);
   else
-    hipLaunchKernelGGL(fp4_tile_weights_kernel<false>, grid_for(chunks), dim3(256), 0, s, codes, rows, cols, KB, chunks, w4);
+    hipLaunchKernelGGL(fp4_tile_weights_kernel<false>, grid_for(chunks), dim3(256), 0, s, codes, rows, cols, KB, chunks,
+                       w4, vec);
   const int64_t ns = sqx_fp4_tiled_scale_bytes(rows, cols, nv ? SQX_FP4_NV : SQX_FP4_MX);
   if (scale_kind == SQX_FP4_SCALE_MX_F32)
     hipLaunchKernelGGL(fp4_tile_scales_kernel<0>, grid_for(ns), dim3(256), 0, s, scales, rows, cols, block, KB, ns, st);

@@ -1,0 +1,145 @@
+"""The vectorised quantizers and tilers against the general ones, and the W8A8 product at its tile edges.
+
+A tensor that starts one element past an aligned address takes the element-wise kernels, the same values at an
+aligned address take the vectorised ones where the sizes allow: codes and scales have to agree bit for bit. The
+int8 product is exact in int32, so its fp32 result is within three roundings (the conversion, the two scales'
+product, the scaled sum) of the integer product in float64.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from tests.conftest import print_case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _shifted(t):
+    """The same values, contiguous, one element past a 16-byte aligned address."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:].copy_(t.reshape(-1))
+    return buf[1:].view(t.shape)
+
+
+def _hostile(rows, cols, dtype, seed):
+    """Rows of normal values, then rows of zeros, signed zeros, denormals, huge and mixed magnitudes, code ties."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(rows, cols, generator=g)
+    x[0] = 0.0
+    x[1 % rows] = -0.0
+    if rows > 8:
+        x[2] *= 1e-40
+        x[3] *= 3e38 if dtype != torch.float16 else 6e4
+        x[4, ::3] *= 1e6
+        x[5] = (torch.arange(cols) % 29 - 14) * 0.5  # halves: every rounding tie
+        x[6, cols // 2] = float("inf")
+        x[7, 0] = -3e38
+        x[8] = 448.0 * (torch.arange(cols) % 2 * 2 - 1)
+    return x.to(dtype).to(DEV)
+
+
+def _same(a, b, what):
+    for i, (u, v) in enumerate(zip(a, b)):
+        u, v = u.detach().contiguous(), v.detach().contiguous()
+        assert u.shape == v.shape and u.dtype == v.dtype, f"{what}[{i}]"
+        if u.dtype == torch.float32:
+            both_nan = torch.isnan(u) & torch.isnan(v)
+            ok = (u.view(torch.int32) == v.view(torch.int32)) | both_nan
+        else:
+            ok = u.view(torch.uint8) == v.view(torch.uint8)
+        assert bool(ok.all()), f"{what}[{i}]: {int((~ok).sum())} of {ok.numel()} differ"
+
+
+def _kv(x):
+    from scratch_llm_amd.quant import fp8_kv_per_head as kv
+
+    r, c = x.shape
+    h = 3 if r % 3 == 0 else 1
+    x4 = x.view(1, h, r // h, c)
+    s = kv.per_head_scale(x4)
+    t = torch.full_like(s, 0.01)  # a static scale: most values saturate
+    return s, kv.per_head_amax(x4), kv.quantize_per_head(x4, s), kv.quantize_per_head(x4, t)
+
+
+def _ops():
+    from scratch_llm_amd.quant import fp8_weights as f8, int4_group as i4, int8 as i8, nvfp4_mxfp4 as f4
+
+    def fp4(q):
+        return [q.codes, q.s_block] + ([q.s_global.reshape(1)] if hasattr(q, "s_global") else [])
+
+    return {
+        "int4": lambda x: i4.quantize_groupwise_int4(x) if x.shape[1] % 128 == 0 else (x,),
+        "int8": lambda x: i8.quantize_symmetric(x, axis=0),
+        "int8_affine": lambda x: i8.quantize_affine(x, axis=0),
+        "fp8": lambda x: f8.quantize_per_channel(x),
+        "mxfp4": lambda x: fp4(f4.mxfp4_quantize(x)),
+        "mxfp4_64": lambda x: fp4(f4.mxfp4_quantize(x, 64)),
+        "nvfp4": lambda x: fp4(f4.nvfp4_quantize(x)),
+        "kv": _kv,
+    }
+
+
+# one chunk, a partial last chunk per wave, several chunks a thread, the register kernels' largest row and one above it
+SHAPES = [(1, 8), (2, 128), (9, 136), (33, 2048), (12, 4104), (10, 14336), (9, 32768), (9, 32776)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("op", ["int4", "int8", "int8_affine", "fp8", "mxfp4", "mxfp4_64", "nvfp4", "kv"])
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_quantizer_same_on_both_paths(rows, cols, op, dtype):
+    print_case("quantizer paths", op, f"{rows}x{cols}", str(dtype))
+    x = _hostile(rows, cols, dtype, rows + cols)
+    f = _ops()[op]
+    assert x.data_ptr() % 16 == 0
+    _same(f(x), f(_shifted(x)), f"{op} {rows}x{cols}")
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 128), (16, 128), (17, 256), (40, 384), (1030, 1152), (33, 4096)])
+def test_tilers_same_on_both_paths(rows, cols):
+    from scratch_llm_amd.quant import fp8_weights as f8, int4_group as i4, int8 as i8, nvfp4_mxfp4 as f4
+
+    print_case("tiler paths", f"{rows}x{cols}")
+    g = torch.Generator().manual_seed(rows + cols)
+    q4 = torch.randint(-8, 8, (rows, cols), generator=g, dtype=torch.int8).to(DEV)
+    s4 = torch.rand(rows, cols // 128, generator=g).to(DEV)
+    p4 = i4.pack_int4(q4.reshape(-1))
+    q8 = torch.randint(-128, 128, (rows, cols), generator=g, dtype=torch.int8).to(DEV)
+    s8 = torch.rand(rows, 1, generator=g).to(DEV)
+    mx = f4.mxfp4_quantize(torch.randn(rows, cols, generator=g).to(DEV))
+    mp, ms = f4.mxfp4_pack_weight(mx)
+    mx2 = type(mx)(_shifted(mx.codes), mx.s_block, mx.shape, mx.n, mx.block)
+    c8, sc8 = f8.quantize_per_channel(torch.randn(rows, cols, generator=g).to(DEV))
+    pairs = {
+        "int4": (i4.tile_int4(q4, s4).wt, i4.tile_int4(_shifted(q4), s4).wt),
+        "int4 packed": (i4.tile_int4(q4, s4).wt, i4.tile_int4_packed(p4, s4, (rows, cols)).wt),
+        "int8": (i8.tile_int8(q8, s8).wt, i8.tile_int8(_shifted(q8), s8).wt),
+        "fp8": (f8.tile_fp8(c8, sc8).wt, f8.tile_fp8(_shifted(c8.view(torch.uint8)).view(c8.dtype), sc8).wt),
+        "fp4": (f4.tile_fp4(mx).wt, f4.tile_fp4(mx2).wt),
+        "fp4 packed": (f4.tile_mxfp4_packed(mp, ms).wt, f4.tile_mxfp4_packed(_shifted(mp), ms).wt),
+    }
+    for name, (a, b) in pairs.items():
+        _same([a], [b], name)
+    assert torch.equal(i8.untile_int8(i8.tile_int8(q8, s8)), q8)
+    assert torch.equal(i4.untile_int4(i4.tile_int4(q4, s4))[0], q4)
+
+
+# one row, partial tiles of both sizes, the larger tile (256 tiles of 128 and more), k below, at and past the ring's
+# stages, a k that is no multiple of 16 (the ragged kernel), and n that is no multiple of 4 (scalar stores)
+@pytest.mark.parametrize("m,n,k", [(1, 1, 16), (3, 70, 64), (64, 64, 128), (65, 129, 1040), (17, 200, 4096), (2049, 2050, 272),
+                                   (2048, 2048, 512), (130, 66, 100), (5, 7, 1), (66, 130, 4095), (300, 4096, 48)])
+def test_w8a8_edges(m, n, k):
+    from scratch_llm_amd.quant import int8 as i8
+
+    print_case("w8a8", f"m={m}", f"n={n}", f"k={k}")
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(DEV)
+    w = torch.randn(n, k, generator=g).to(DEV)
+    y = i8.w8a8_linear(x, w).double().cpu().numpy()
+    (qx, sx), (qw, sw) = i8.quantize_symmetric(x, axis=0), i8.quantize_symmetric(w, axis=0)
+    acc = qx.double().cpu().numpy() @ qw.double().cpu().numpy().T  # whole numbers below 2**53: exact
+    ref = acc * sx.double().cpu().numpy().reshape(-1, 1) * sw.double().cpu().numpy().reshape(1, -1)
+    assert np.all(np.abs(y - ref) <= 3.01 * 2.0**-24 * np.abs(ref))
