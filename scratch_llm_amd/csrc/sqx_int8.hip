@@ -9,6 +9,7 @@
 // Tiled int8 layout (the weight-only linear): block (t, kb) = 1 KiB covering 16 rows x 64 columns;
 // lane L owns the 16 codes of row 16t + (L & 15), columns kb*64 + 16(L >> 4) + e, stored as
 // u = q + 128 in byte e. Per-row fp32 scales are read in the epilogue.
+#include "sqx_quant.h"
 #include "sqx_skinny.h"
 
 namespace sqx {
@@ -42,22 +43,27 @@ __device__ inline float nmin(float m, float v) { return (v < m || v != v) ? v : 
 //              z = clamp(rint(rd(-lo / s)), 0, 255)
 // ----------------------------------------------------------------------------------------------
 template <int DT, int OP>
-__device__ inline void finish_stats(float a, float b, float eps, void* s_out, void* z_out, int64_t i) {
+__device__ inline void slice_params(float a, float b, float eps, float& s, float& z) {
   const float e = rd<DT>(eps);
+  z = 0.0f;
   if (OP == 0) {
-    float s = rd<DT>(__fdiv_rn(a, 127.0f));
+    s = rd<DT>(__fdiv_rn(a, 127.0f));
     if (s < e) s = e;
-    store_dt<DT>(s_out, i, s);
   } else {
     const float lo = a < 0.0f || a != a ? a : 0.0f;  // torch.minimum(x, 0) propagates NaN
     const float hi = b > 0.0f || b != b ? b : 0.0f;
-    float s = rd<DT>(__fdiv_rn(rd<DT>(hi - lo), 255.0f));
+    s = rd<DT>(__fdiv_rn(rd<DT>(hi - lo), 255.0f));
     if (s < e) s = e;
-    float z = __builtin_rintf(rd<DT>(__fdiv_rn(-lo, s)));
+    z = __builtin_rintf(rd<DT>(__fdiv_rn(-lo, s)));
     z = fminf(fmaxf(z, 0.0f), 255.0f);
-    store_dt<DT>(s_out, i, s);
-    store_dt<DT>(z_out, i, z);
   }
+}
+template <int DT, int OP>
+__device__ inline void finish_stats(float a, float b, float eps, void* s_out, void* z_out, int64_t i) {
+  float s, z;
+  slice_params<DT, OP>(a, b, eps, s, z);
+  store_dt<DT>(s_out, i, s);
+  if (OP == 1) store_dt<DT>(z_out, i, z);
 }
 
 // One workgroup per kept index b (C >= 32 or A*C large): reduces x[a, b, c] over a and c.
@@ -187,6 +193,76 @@ __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ 
   }
 }
 
+// The same two steps for the rows of a [B, C] matrix (A = 1), in one pass: the row stays in registers between
+// its statistics and its codes. 256 threads a row, 8 consecutive elements per thread and chunk (chunk c of the
+// row is thread c % 256's). w8a8_linear quantizes both operands on every call: 14336 x 4096 in bf16 took 184 us in
+// two passes (element loads, 64-bit divisions for the slice index, an IEEE division per element), 37.7 us (4.7 TB/s)
+// in one.
+template <int DT>
+__device__ inline float rd_fast(float v) {  // rd without its NaN case (NaN stays NaN)
+  if (DT == SQX_DTYPE_BF16) return bf16_lo(ActBF16::pack_rne(v, 0.0f));
+  return rd<DT>(v);
+}
+
+template <int DT, int OP, int NCH>
+__global__ __launch_bounds__(256) void quantize_rows_kernel(const void* __restrict__ x, int64_t C, float eps,
+                                                            void* __restrict__ s_out, void* __restrict__ z_out,
+                                                            uint8_t* __restrict__ q) {
+  __shared__ float red[2][4];
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int nch = static_cast<int>(C / 8);
+  float v[NCH][8];
+  float m0 = OP == 0 ? 0.0f : INFINITY, m1 = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+    if (tid + 256 * i < nch) load8_f32(x, DT, row * C + 8 * (tid + 256 * i), v[i]);
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+    if (tid + 256 * i < nch) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (OP == 0) m0 = nmax(m0, fabsf(v[i][e]));
+        else m0 = nmin(m0, v[i][e]), m1 = nmax(m1, v[i][e]);
+      }
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    if (OP == 0) m0 = nmax(m0, __shfl_xor(m0, o, 64));
+    else m0 = nmin(m0, __shfl_xor(m0, o, 64)), m1 = nmax(m1, __shfl_xor(m1, o, 64));
+  }
+  if ((tid & 63) == 0) red[0][tid >> 6] = m0, red[1][tid >> 6] = m1;
+  __syncthreads();
+  m0 = red[0][0], m1 = red[1][0];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    if (OP == 0) m0 = nmax(m0, red[0][w]);
+    else m0 = nmin(m0, red[0][w]), m1 = nmax(m1, red[1][w]);
+  }
+  float sv, zv;
+  slice_params<DT, OP>(m0, m1, eps, sv, zv);
+  if (tid == 0) {
+    store_dt<DT>(s_out, row, sv);
+    if (OP == 1) store_dt<DT>(z_out, row, zv);
+  }
+  const SharedDiv sd = shared_div(sv);
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+    if (tid + 256 * i < nch) {
+      uint32_t w[2] = {0u, 0u};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float t = rd_fast<DT>(div_by(sd, v[i][e]));
+        float r;
+        if (OP == 0) r = fminf(fmaxf(__builtin_rintf(t), -127.0f), 127.0f);
+        else r = fminf(fmaxf(__builtin_rintf(rd_fast<DT>(t + zv)), 0.0f), 255.0f);
+        const int c = static_cast<int>(r == r ? r : 0.0f);
+        w[e >> 2] |= (static_cast<uint32_t>(c) & 0xffu) << (8 * (e & 3));
+      }
+      *reinterpret_cast<u32x2v_t*>(q + row * C + 8 * (tid + 256 * i)) = u32x2v_t{w[0], w[1]};
+    }
+}
+
 // symmetric: rd(q * s); affine: rd(rd(q - z) * s) (int8.py:127-129, 174-176), in the scale dtype.
 template <int DT, int OP>
 __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restrict__ q, int64_t n, int64_t B,
@@ -204,45 +280,136 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
 
 // ----------------------------------------------------------------------------------------------
 // w8a8_linear (int8.py:189-213): acc = q_x @ q_w^T in int32 (exact), y = fp32(acc) * (s_x[m] * s_w[n])
-// with the scale product in the promoted scale dtype PD. One wave per 16x16 output tile, 4 waves per
-// workgroup (32x32), v_mfma_i32_16x16x64_i8: lanes of group g = lane >> 4 carry the same 16 columns
-// of A (row lane & 15) and B (column lane & 15), so each product pairs matching k.
+// with the scale product in the promoted scale dtype PD, on v_mfma_i32_16x16x64_i8.
+//
+// A workgroup of four waves owns a T x T output tile (T = 64 or 128), each wave a quarter. A stage covers 128 k of
+// the T rows of either operand, 128 bytes a row, copied by buffer loads that write LDS directly into a ring of NS
+// stages; 16-byte chunk c of row r lies at slot c ^ (r & 7), so the 16 rows of a fragment read touch distinct
+// banks. w is the MFMA's first operand: a lane's four accumulators are four consecutive columns of one row.
+// The 64-row tile takes grids that 128-row tiles would leave below one workgroup per CU. A form without LDS,
+// one 16 x 16 tile a wave, took 61 us for 256 x 4096 x 4096. The linear with both quantizers, before and now: 132 and
+// 39 us at that size, 536 and 94 us at 2048 x 4096 x 4096, 976 and 192 us at 1024 x 14336 x 4096.
 // ----------------------------------------------------------------------------------------------
 typedef int i32x4_t __attribute__((__vector_size__(4 * sizeof(int))));
 
-template <int PD>
-__global__ __launch_bounds__(256) void w8a8_kernel(const int8_t* __restrict__ qx, const int8_t* __restrict__ qw,
+template <int PD, int T, int NS>
+__global__ __launch_bounds__(256, 2) void w8a8_kernel(const int8_t* __restrict__ qx, const int8_t* __restrict__ qw,
                                                    const void* __restrict__ sx, int sx_dt, const void* __restrict__ sw,
-                                                   int sw_dt, float* __restrict__ y, int M, int N, int K) {
+                                                   int sw_dt, float* __restrict__ y, int M, int N, int K, int tiles_m) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
+  constexpr int kStage = 2 * T * 128;   // x rows, then w rows
+  constexpr int CPW = 2 * T / 8 / 4;    // 1 KiB copies (8 rows) per wave and stage
+  constexpr int F = T / 32;             // 16-row fragments of either operand per wave
+  constexpr uint32_t kNone = 0x80000000u;  // past either buffer (both below 2 GiB): zeros, no memory traffic
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // consecutive workgroups take the row tiles of one column tile, so they share w's rows
+  const int m0 = (blockIdx.x % tiles_m) * T, n0 = (blockIdx.x / tiles_m) * T;
+  const rsrc_t xr = make_rsrc(qx, (uint32_t)M * (uint32_t)K);
+  const rsrc_t wr = make_rsrc(qw, (uint32_t)N * (uint32_t)K);
+  const bool is_w = wave >= 2;  // waves 0, 1 copy x's rows, 2, 3 w's
+  const rsrc_t cr = is_w ? wr : xr;
+  const int lim = is_w ? N - n0 : M - m0;
+  const uint32_t row_base = (uint32_t)(is_w ? n0 : m0) * (uint32_t)K;
+  const int S = (K + 127) / 128;
+  auto issue = [&](int s, int slot) {
+    uint8_t* dst = smem8 + slot * kStage + wave * CPW * 1024;
+#pragma unroll
+    for (int j = 0; j < CPW; ++j) {
+      const int r = ((wave & 1) * CPW + j) * 8 + (lane >> 3);
+      const int c = 128 * s + 16 * ((lane & 7) ^ (r & 7));
+      const uint32_t off = (r < lim) & (c < K) ? row_base + (uint32_t)r * (uint32_t)K + (uint32_t)c : kNone;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(cr, (lds_void*)(dst + j * 1024), 16, off, 0, 0, 0);
+    }
+  };
+  i32x4_t acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = i32x4_t{0, 0, 0, 0};
+  const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+  const int r = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s)
+    if (s < S) issue(s, s);
+  int slot = 0;
+  for (int s = 0; s < S; ++s) {
+    // stage s has landed for this wave (the NS - 2 after it may be in flight), then for all; every wave has also
+    // read stage s - 1 (its MFMAs waited for the reads), whose slot the next copies take
+    if (s + NS - 2 < S) wait_vmcnt<CPW * (NS - 2)>();
+    else wait_vmcnt<0>();
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (s + NS - 1 < S) issue(s + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+    const uint8_t* xb = smem8 + slot * kStage;
+    const uint8_t* wb = xb + T * 128;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4_t a[F], b[F];
+      const int sl = ((4 * h + g) ^ (r & 7)) * 16;
+#pragma unroll
+      for (int i = 0; i < F; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(xb + (wm + 16 * i + r) * 128 + sl);
+#pragma unroll
+      for (int i = 0; i < F; ++i) b[i] = *reinterpret_cast<const u32x4_t*>(wb + (wn + 16 * i + r) * 128 + sl);
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4_t, b[j]),
+                                                            __builtin_bit_cast(i32x4_t, a[i]), acc[i][j], 0, 0, 0);
+    }
+    slot = slot == NS - 1 ? 0 : slot + 1;
+  }
+  // acc[i][j][e] is y[m0 + wm + 16i + (l & 15)][n0 + wn + 16j + 4(l >> 4) + e]
+  const bool vec = N % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    const int m = m0 + wm + 16 * i + r;
+    if (m >= M) continue;
+    const float sm = load_as_f32(sx, sx_dt, m);
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const int n = n0 + wn + 16 * j + 4 * g;
+      if (n >= N) continue;
+      f32x4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = static_cast<float>(acc[i][j][e]) * rd<PD>(sm * load_as_f32(sw, sw_dt, min(n + e, N - 1)));
+      float* dst = y + (int64_t)m * N + n;
+      if (vec) {
+        *reinterpret_cast<f32x4_t*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) dst[e] = v[e];
+      }
+    }
+  }
+}
+
+// The same product for rows that are not a multiple of 16 bytes: one wave per 16 x 16 tile, element loads.
+template <int PD>
+__global__ __launch_bounds__(256) void w8a8_ragged_kernel(const int8_t* __restrict__ qx, const int8_t* __restrict__ qw,
+                                                          const void* __restrict__ sx, int sx_dt,
+                                                          const void* __restrict__ sw, int sw_dt, float* __restrict__ y,
+                                                          int M, int N, int K) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int m0 = blockIdx.y * 32 + (wave >> 1) * 16;
   const int n0 = blockIdx.x * 32 + (wave & 1) * 16;
   const int r = lane & 15, g = lane >> 4;
   const int am = m0 + r, bn = n0 + r;
-  const rsrc_t ar = make_rsrc(qx, (uint32_t)M * (uint32_t)K);
-  const rsrc_t br = make_rsrc(qw, (uint32_t)N * (uint32_t)K);
   i32x4_t acc = {0, 0, 0, 0};
-  const bool kfull = K % 16 == 0;
   for (int k0 = 0; k0 < K; k0 += 64) {
     const int kk = k0 + 16 * g;
-    u32x4_t a, b;
-    if (kfull) {
-      // rows at or beyond M / N read zero (past the end of the buffer); columns at or beyond K are
-      // the next row's: masked below
-      a = kk < K && am < M ? bload128(ar, (uint32_t)(am * K + kk), 0u) : u32x4_t{0u, 0u, 0u, 0u};
-      b = kk < K && bn < N ? bload128(br, (uint32_t)(bn * K + kk), 0u) : u32x4_t{0u, 0u, 0u, 0u};
-    } else {
-      uint32_t av[4] = {0u, 0u, 0u, 0u}, bv[4] = {0u, 0u, 0u, 0u};
-      for (int e = 0; e < 16; ++e) {
-        if (kk + e < K) {
-          if (am < M) av[e >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(qx[(int64_t)am * K + kk + e])) << (8 * (e & 3));
-          if (bn < N) bv[e >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(qw[(int64_t)bn * K + kk + e])) << (8 * (e & 3));
-        }
+    uint32_t av[4] = {0u, 0u, 0u, 0u}, bv[4] = {0u, 0u, 0u, 0u};
+    for (int e = 0; e < 16; ++e) {
+      if (kk + e < K) {
+        if (am < M) av[e >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(qx[(int64_t)am * K + kk + e])) << (8 * (e & 3));
+        if (bn < N) bv[e >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(qw[(int64_t)bn * K + kk + e])) << (8 * (e & 3));
       }
-      a = u32x4_t{av[0], av[1], av[2], av[3]};
-      b = u32x4_t{bv[0], bv[1], bv[2], bv[3]};
     }
+    const u32x4_t a = {av[0], av[1], av[2], av[3]}, b = {bv[0], bv[1], bv[2], bv[3]};
     acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4_t, a), __builtin_bit_cast(i32x4_t, b), acc,
                                                 0, 0, 0);
   }
@@ -332,24 +499,28 @@ struct WInt8 {
   static const float* out_scales(const Args& a) { return a.scale; }
 };
 
-// One thread per output dword of the tiled int8 weight.
+// One thread per output dword of the tiled int8 weight. vec: the four codes are one aligned dword.
 __global__ __launch_bounds__(256) void int8_tile_kernel(const int8_t* __restrict__ q, int64_t rows, int64_t cols,
-                                                        int64_t KB, int64_t n_dwords, uint32_t* __restrict__ wt) {
+                                                        int64_t KB, int64_t n_dwords, uint32_t* __restrict__ wt, int vec) {
   const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (d >= n_dwords) return;
   const int i = static_cast<int>(d & 3);
   const int L = static_cast<int>((d >> 2) & 63);
-  const int64_t blk = d >> 8;
-  const int64_t t = blk / KB;
+  const uint32_t blk = static_cast<uint32_t>(d >> 8);  // blocks of 1 KiB: below 2**32
+  const int64_t t = blk / static_cast<uint32_t>(KB);
   const int64_t kb = blk - t * KB;
   const int64_t r = 16 * t + (L & 15);
   const int64_t c0 = kb * 64 + 16 * (L >> 4) + 4 * i;
   uint32_t word = 0;
+  if (vec && r < rows && c0 + 4 <= cols) {
+    word = *reinterpret_cast<const uint32_t*>(q + r * cols + c0) ^ 0x80808080u;  // q + 128 in every byte
+  } else {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int64_t c = c0 + e;
-    const uint32_t u = (r < rows && c < cols) ? static_cast<uint32_t>(q[r * cols + c] + 128) : 128u;
-    word |= (u & 0xffu) << (8 * e);
+    for (int e = 0; e < 4; ++e) {
+      const int64_t c = c0 + e;
+      const uint32_t u = (r < rows && c < cols) ? static_cast<uint32_t>(q[r * cols + c] + 128) : 128u;
+      word |= (u & 0xffu) << (8 * e);
+    }
   }
   wt[d] = word;
 }
@@ -431,6 +602,27 @@ static int int8_quantize(const void* x, int dtype, int64_t A, int64_t B, int64_t
   SQX_REQUIRE(x && q && s && (OP == 0 || z), SQX_E_ARG, "%s: null pointer", fn);
   SQX_REQUIRE(B == 1 || B < ((int64_t)1 << 31), SQX_E_ARG, "%s: kept axis too long", fn);
   hipStream_t st = as_stream(stream);
+  // rows of a matrix: one pass, for rows of whole aligned 8-element chunks that fit a workgroup's registers
+  if (A == 1 && B > 1 && C % 8 == 0 && C <= 16 * 2048 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(q) % 8 == 0) {
+    const dim3 grid(static_cast<unsigned>(B));
+#define SQX_QR(DT, N) hipLaunchKernelGGL((quantize_rows_kernel<DT, OP, N>), grid, dim3(256), 0, st, x, C, eps, s, z, q)
+#define SQX_QRN(DT)                  \
+  do {                               \
+    if (C <= 2048) SQX_QR(DT, 1);    \
+    else if (C <= 4096) SQX_QR(DT, 2);  \
+    else if (C <= 8192) SQX_QR(DT, 4);  \
+    else if (C <= 16384) SQX_QR(DT, 8); \
+    else SQX_QR(DT, 16);             \
+  } while (0)
+    if (dtype == SQX_DTYPE_F32) SQX_QRN(SQX_DTYPE_F32);
+    else if (dtype == SQX_DTYPE_BF16) SQX_QRN(SQX_DTYPE_BF16);
+    else SQX_QRN(SQX_DTYPE_F16);
+#undef SQX_QRN
+#undef SQX_QR
+    SQX_LAUNCH_CHECK(fn);
+    return SQX_OK;
+  }
   int rc = int8_stats<OP>(x, dtype, A, B, C, eps, s, z, workspace, workspace_bytes, st, fn);
   if (rc) return rc;
   const int64_t n = A * B * C;
@@ -494,6 +686,7 @@ extern "C" int sqx_w8a8_gemm(const int8_t* qx, const void* sx, int sx_dtype, con
   SQX_REQUIRE(is_float_dtype(sx_dtype) && is_float_dtype(sw_dtype), SQX_E_ARG, "sqx_w8a8_gemm: bad scale dtype");
   SQX_REQUIRE(m >= 0 && n >= 0 && k >= 1 && m * k < ((int64_t)1 << 31) && n * k < ((int64_t)1 << 31), SQX_E_ARG,
               "sqx_w8a8_gemm: bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
+  SQX_REQUIRE(ceil_div(m, 64) * ceil_div(n, 64) < ((int64_t)1 << 31), SQX_E_ARG, "sqx_w8a8_gemm: too many output tiles");
   SQX_REQUIRE(k <= 131072, SQX_E_ARG, "sqx_w8a8_gemm: k=%lld may overflow the int32 accumulator", (long long)k);
   if (m == 0 || n == 0) return SQX_OK;
   SQX_REQUIRE(qx && sx && qw && sw && y, SQX_E_ARG, "sqx_w8a8_gemm: null pointer");
@@ -501,15 +694,33 @@ extern "C" int sqx_w8a8_gemm(const int8_t* qx, const void* sx, int sx_dtype, con
               SQX_E_ARG, "sqx_w8a8_gemm: qx and qw must be 16-byte aligned");
   // the scale product is taken in the promoted dtype of the two scales (torch type promotion)
   const int pd = sx_dtype == sw_dtype ? sx_dtype : SQX_DTYPE_F32;
-  const dim3 grid(static_cast<unsigned>(ceil_div(n, 32)), static_cast<unsigned>(ceil_div(m, 32)));
   hipStream_t st = as_stream(stream);
   const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
-  if (pd == SQX_DTYPE_F32)
-    hipLaunchKernelGGL(w8a8_kernel<SQX_DTYPE_F32>, grid, dim3(256), 0, st, qx, qw, sx, sx_dtype, sw, sw_dtype, y, M, N, K);
-  else if (pd == SQX_DTYPE_BF16)
-    hipLaunchKernelGGL(w8a8_kernel<SQX_DTYPE_BF16>, grid, dim3(256), 0, st, qx, qw, sx, sx_dtype, sw, sw_dtype, y, M, N, K);
-  else
-    hipLaunchKernelGGL(w8a8_kernel<SQX_DTYPE_F16>, grid, dim3(256), 0, st, qx, qw, sx, sx_dtype, sw, sw_dtype, y, M, N, K);
+  hipError_t e = hipSuccess;
+  auto go = [&](auto kern, int T, int stages) {
+    const int64_t tm = ceil_div(m, T), tn = ceil_div(n, T);
+    const int lds = stages * 2 * T * 128;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e == hipSuccess)
+      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tm * tn)), dim3(256), static_cast<size_t>(lds), st, qx, qw, sx,
+                         sx_dtype, sw, sw_dtype, y, M, N, K, static_cast<int>(tm));
+  };
+  // 128 x 128 tiles once they fill the 256 CUs (1024 x 4096 x 4096), 64 x 64 below
+  const bool big = ceil_div(m, 128) * ceil_div(n, 128) >= 256;
+#define SQX_W8(PD)                                                                                                    \
+  do {                                                                                                                \
+    if (k % 16 != 0)                                                                                                  \
+      hipLaunchKernelGGL(w8a8_ragged_kernel<PD>,                                                                       \
+                         dim3(static_cast<unsigned>(ceil_div(n, 32)), static_cast<unsigned>(ceil_div(m, 32))), dim3(256), \
+                         0, st, qx, qw, sx, sx_dtype, sw, sw_dtype, y, M, N, K);                                       \
+    else if (big) go(w8a8_kernel<PD, 128, 4>, 128, 4);                                                                 \
+    else go(w8a8_kernel<PD, 64, 4>, 64, 4);                                                                            \
+  } while (0)
+  if (pd == SQX_DTYPE_F32) SQX_W8(SQX_DTYPE_F32);
+  else if (pd == SQX_DTYPE_BF16) SQX_W8(SQX_DTYPE_BF16);
+  else SQX_W8(SQX_DTYPE_F16);
+#undef SQX_W8
+  SQX_REQUIRE(e == hipSuccess, SQX_E_HIP, "sqx_w8a8_gemm: launch failed: %s", hipGetErrorString(e));
   SQX_LAUNCH_CHECK("sqx_w8a8_gemm");
   return SQX_OK;
 }
@@ -526,7 +737,7 @@ extern "C" int sqx_int8_tile(const int8_t* q, int64_t rows, int64_t cols, uint8_
   const int64_t KB = ceil_div(cols, 64);
   const int64_t nd = ceil_div(rows, 16) * KB * 256;
   hipLaunchKernelGGL(int8_tile_kernel, grid_for(nd), dim3(256), 0, as_stream(stream), q, rows, cols, KB, nd,
-                     reinterpret_cast<uint32_t*>(wt));
+                     reinterpret_cast<uint32_t*>(wt), cols % 4 == 0 && reinterpret_cast<uintptr_t>(q) % 4 == 0);
   SQX_LAUNCH_CHECK("sqx_int8_tile");
   return SQX_OK;
 }
