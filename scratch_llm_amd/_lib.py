@@ -148,6 +148,8 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "sqx_int8_dequantize_sym": (_c_i, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i, _c_p, _c_p]),
     "sqx_int8_dequantize_affine": (_c_i, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_i, _c_p, _c_p]),
     "sqx_w8a8_gemm": (_c_i, [_c_p, _c_p, _c_i, _c_p, _c_p, _c_i, _c_p, _c_i64, _c_i64, _c_i64, _c_p]),
+    "sqx_w8a8_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "sqx_w8a8_linear": (_c_i, [_c_p, _c_p, _c_i, ctypes.c_float, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p]),
     "sqx_int8_tiled_weight_bytes": (_c_i64, [_c_i64, _c_i64]),
     "sqx_int8_tile": (_c_i, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),
     "sqx_int8_linear": (_c_i, [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_p]),

@@ -197,7 +197,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ 
 // its statistics and its codes. 256 threads a row, 8 consecutive elements per thread and chunk (chunk c of the
 // row is thread c % 256's). w8a8_linear quantizes both operands on every call: 14336 x 4096 in bf16 took 184 us in
 // two passes (element loads, 64-bit divisions for the slice index, an IEEE division per element), 37.7 us (4.7 TB/s)
-// in one.
+// in one. Rows from B1 on come from a second matrix x2 of the same width, so w8a8_linear's two operands take one
+// launch.
 template <int DT>
 __device__ inline float rd_fast(float v) {  // rd without its NaN case (NaN stays NaN)
   if (DT == SQX_DTYPE_BF16) return bf16_lo(ActBF16::pack_rne(v, 0.0f));
@@ -205,7 +206,8 @@ __device__ inline float rd_fast(float v) {  // rd without its NaN case (NaN stay
 }
 
 template <int DT, int OP, int NCH>
-__global__ __launch_bounds__(256) void quantize_rows_kernel(const void* __restrict__ x, int64_t C, float eps,
+__global__ __launch_bounds__(256) void quantize_rows_kernel(const void* __restrict__ x, const void* __restrict__ x2,
+                                                            int64_t B1, int64_t C, float eps,
                                                             void* __restrict__ s_out, void* __restrict__ z_out,
                                                             uint8_t* __restrict__ q) {
   __shared__ float red[2][4];
@@ -214,9 +216,11 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* __restri
   const int nch = static_cast<int>(C / 8);
   float v[NCH][8];
   float m0 = OP == 0 ? 0.0f : INFINITY, m1 = -INFINITY;
+  const void* src = row < B1 ? x : x2;
+  const int64_t src0 = (row < B1 ? row : row - B1) * C;
 #pragma unroll
   for (int i = 0; i < NCH; ++i)
-    if (tid + 256 * i < nch) load8_f32(x, DT, row * C + 8 * (tid + 256 * i), v[i]);
+    if (tid + 256 * i < nch) load8_f32(src, DT, src0 + 8 * (tid + 256 * i), v[i]);
 #pragma unroll
   for (int i = 0; i < NCH; ++i)
     if (tid + 256 * i < nch) {
@@ -289,6 +293,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
 // The 64-row tile takes grids that 128-row tiles would leave below one workgroup per CU. A form without LDS,
 // one 16 x 16 tile a wave, took 61 us for 256 x 4096 x 4096. The linear with both quantizers, before and now: 132 and
 // 39 us at that size, 536 and 94 us at 2048 x 4096 x 4096, 976 and 192 us at 1024 x 14336 x 4096.
+// (29 us at that size since w8a8_tile_of below and the one quantizer launch.)
 // ----------------------------------------------------------------------------------------------
 typedef int i32x4_t __attribute__((__vector_size__(4 * sizeof(int))));
 
@@ -613,6 +618,30 @@ static int int8_stats(const void* x, int dtype, int64_t A, int64_t B, int64_t C,
 
 extern "C" int64_t sqx_int8_workspace_bytes(void) { return (int64_t)kStatParts * 8; }
 
+// One pass over the B rows of x (from row B1 on: of x2), for rows of whole aligned 8-element chunks that fit a
+// workgroup's registers.
+constexpr int64_t kQuantRowsMaxC = 16 * 2048;
+template <int OP>
+static void launch_quantize_rows(const void* x, const void* x2, int64_t B1, int64_t B, int dtype, int64_t C, float eps,
+                                 uint8_t* q, void* s, void* z, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(B));
+#define SQX_QR(DT, N) \
+  hipLaunchKernelGGL((quantize_rows_kernel<DT, OP, N>), grid, dim3(256), 0, st, x, x2, B1, C, eps, s, z, q)
+#define SQX_QRN(DT)                     \
+  do {                                  \
+    if (C <= 2048) SQX_QR(DT, 1);       \
+    else if (C <= 4096) SQX_QR(DT, 2);  \
+    else if (C <= 8192) SQX_QR(DT, 4);  \
+    else if (C <= 16384) SQX_QR(DT, 8); \
+    else SQX_QR(DT, 16);                \
+  } while (0)
+  if (dtype == SQX_DTYPE_F32) SQX_QRN(SQX_DTYPE_F32);
+  else if (dtype == SQX_DTYPE_BF16) SQX_QRN(SQX_DTYPE_BF16);
+  else SQX_QRN(SQX_DTYPE_F16);
+#undef SQX_QRN
+#undef SQX_QR
+}
+
 template <int OP>
 static int int8_quantize(const void* x, int dtype, int64_t A, int64_t B, int64_t C, float eps, uint8_t* q, void* s,
                          void* z, void* workspace, int64_t workspace_bytes, sqx_stream_t stream, const char* fn) {
@@ -623,23 +652,9 @@ static int int8_quantize(const void* x, int dtype, int64_t A, int64_t B, int64_t
   SQX_REQUIRE(B == 1 || B < ((int64_t)1 << 31), SQX_E_ARG, "%s: kept axis too long", fn);
   hipStream_t st = as_stream(stream);
   // rows of a matrix: one pass, for rows of whole aligned 8-element chunks that fit a workgroup's registers
-  if (A == 1 && B > 1 && C % 8 == 0 && C <= 16 * 2048 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+  if (A == 1 && B > 1 && C % 8 == 0 && C <= kQuantRowsMaxC && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 8 == 0) {
-    const dim3 grid(static_cast<unsigned>(B));
-#define SQX_QR(DT, N) hipLaunchKernelGGL((quantize_rows_kernel<DT, OP, N>), grid, dim3(256), 0, st, x, C, eps, s, z, q)
-#define SQX_QRN(DT)                  \
-  do {                               \
-    if (C <= 2048) SQX_QR(DT, 1);    \
-    else if (C <= 4096) SQX_QR(DT, 2);  \
-    else if (C <= 8192) SQX_QR(DT, 4);  \
-    else if (C <= 16384) SQX_QR(DT, 8); \
-    else SQX_QR(DT, 16);             \
-  } while (0)
-    if (dtype == SQX_DTYPE_F32) SQX_QRN(SQX_DTYPE_F32);
-    else if (dtype == SQX_DTYPE_BF16) SQX_QRN(SQX_DTYPE_BF16);
-    else SQX_QRN(SQX_DTYPE_F16);
-#undef SQX_QRN
-#undef SQX_QR
+    launch_quantize_rows<OP>(x, nullptr, B, B, dtype, C, eps, q, s, z, st);
     SQX_LAUNCH_CHECK(fn);
     return SQX_OK;
   }
@@ -743,6 +758,33 @@ extern "C" int sqx_w8a8_gemm(const int8_t* qx, const void* sx, int sx_dtype, con
   SQX_REQUIRE(e == hipSuccess, SQX_E_HIP, "sqx_w8a8_gemm: launch failed: %s", hipGetErrorString(e));
   SQX_LAUNCH_CHECK("sqx_w8a8_gemm");
   return SQX_OK;
+}
+
+extern "C" int64_t sqx_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+  // int8 rows of x, then of w, then their scales (at most fp32)
+  return k % 16 == 0 && k <= kQuantRowsMaxC && m > 0 && n > 0 && k > 0 && m + n < ((int64_t)1 << 31) &&
+                 m * k < ((int64_t)1 << 31) && n * k < ((int64_t)1 << 31)
+             ? (m + n) * (k + 4)
+             : -1;
+}
+
+extern "C" int sqx_w8a8_linear(const void* x, const void* w, int dtype, float eps, float* y, int64_t m, int64_t n, int64_t k,
+                               void* ws, int64_t ws_bytes, sqx_stream_t stream) {
+  SQX_REQUIRE(is_float_dtype(dtype), SQX_E_ARG, "sqx_w8a8_linear: unsupported dtype %d", dtype);
+  const int64_t need = sqx_w8a8_workspace_bytes(m, n, k);
+  SQX_REQUIRE(need > 0, SQX_E_ARG, "sqx_w8a8_linear: bad shape m=%lld n=%lld k=%lld (k %% 16 == 0, k <= %lld)", (long long)m,
+              (long long)n, (long long)k, (long long)kQuantRowsMaxC);
+  SQX_REQUIRE(x && w && y && ws, SQX_E_ARG, "sqx_w8a8_linear: null pointer");
+  SQX_REQUIRE(ws_bytes >= need, SQX_E_SPACE, "sqx_w8a8_linear: the workspace needs %lld bytes", (long long)need);
+  SQX_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(ws) % 16 == 0,
+              SQX_E_ARG, "sqx_w8a8_linear: x, w and the workspace must be 16-byte aligned");
+  auto* q = static_cast<uint8_t*>(ws);
+  uint8_t* s = q + (m + n) * k;
+  launch_quantize_rows<0>(x, w, m, m + n, dtype, k, eps, q, s, nullptr, as_stream(stream));
+  SQX_LAUNCH_CHECK("sqx_w8a8_linear");
+  return sqx_w8a8_gemm(reinterpret_cast<const int8_t*>(q), s, dtype, reinterpret_cast<const int8_t*>(q + m * k),
+                       s + m * (dtype == SQX_DTYPE_F32 ? 4 : 2), dtype, y, m, n, k, stream);
 }
 
 extern "C" int64_t sqx_int8_tiled_weight_bytes(int64_t rows, int64_t cols) {

@@ -213,6 +213,20 @@ def w8a8_linear(x: Tensor, w: Tensor) -> Tensor:
     ``acc.to(fp32) * (s_x * s_w)``. ``x`` is ``[..., in]``, ``w`` is ``[out, in]``."""
     *batch, in_features = x.shape
     x2d = x.reshape(-1, in_features)
+    # both operands quantized in one launch and one call, where they have one dtype and whole aligned 16-byte rows that
+    # fit the quantizer's registers (256 x 4096 x 4096: 40.7 us in three calls, bound by the host, 29.2 in one)
+    if x.dtype == w.dtype and x.dtype in _DTYPES and x.is_cuda and w.device == x.device and w.shape[1:] == (in_features,):
+        lib = _lib.load()
+        m, n = x2d.shape[0], w.shape[0]
+        xc, wc = x2d.detach().contiguous(), w.detach().contiguous()
+        nb = int(lib.sqx_w8a8_workspace_bytes(m, n, in_features))
+        if nb > 0 and xc.data_ptr() % 16 == 0 and wc.data_ptr() % 16 == 0:
+            ws = torch.empty(nb, dtype=torch.uint8, device=x.device)
+            y = torch.empty(*batch, n, dtype=torch.float32, device=x.device)
+            with torch.cuda.device(x.device):
+                _lib.check(lib.sqx_w8a8_linear(xc.data_ptr(), wc.data_ptr(), _lib.sqx_dtype(x.dtype), 1e-12, y.data_ptr(), m,
+                                               n, in_features, ws.data_ptr(), nb, _lib.stream_ptr(x.device)), "w8a8_linear")
+            return y
     q_x, s_x = quantize_symmetric(x2d, axis=0)
     q_w, s_w = quantize_symmetric(w, axis=0)
     m, n, k = q_x.shape[0], q_w.shape[0], in_features

@@ -143,3 +143,37 @@ def test_w8a8_edges(m, n, k):
     acc = qx.double().cpu().numpy() @ qw.double().cpu().numpy().T  # whole numbers below 2**53: exact
     ref = acc * sx.double().cpu().numpy().reshape(-1, 1) * sw.double().cpu().numpy().reshape(1, -1)
     assert np.all(np.abs(y - ref) <= 3.01 * 2.0**-24 * np.abs(ref))
+
+
+# the call that quantizes both operands in one launch against the quantizer and the product called one by one, at the
+# edges of its row chunks (2048, 4096, .. columns), and the forms that it does not take (k % 16, unaligned, two dtypes)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 16), (1, 33, 2048), (5, 3, 2064), (33, 70, 4112), (2, 9, 16400), (3, 2, 32768),
+                                   (3, 2, 32784), (4, 6, 100), (130, 515, 256)])
+def test_w8a8_one_launch(m, n, k, dtype):
+    from scratch_llm_amd import _lib
+    from scratch_llm_amd.quant import int8 as i8
+
+    print_case("w8a8 one launch", f"m={m}", f"n={n}", f"k={k}", f"dtype={dtype}")
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k, generator=g).to(dtype), torch.randn(n, k, generator=g).to(dtype)
+    w[0] = 0.0  # the scale is eps
+    if m > 2:
+        x[1, 3], x[2, 5] = float("nan"), float("inf")
+    x, w = x.to(DEV), w.to(DEV)
+
+    def parts(x, w):
+        (qx, sx), (qw, sw) = i8.quantize_symmetric(x, axis=0), i8.quantize_symmetric(w, axis=0)
+        y = torch.empty(m, n, device=DEV)
+        _lib.check(_lib.load().sqx_w8a8_gemm(qx.data_ptr(), sx.data_ptr(), _lib.sqx_dtype(sx.dtype), qw.data_ptr(),
+                                             sw.data_ptr(), _lib.sqx_dtype(sw.dtype), y.data_ptr(), m, n, k,
+                                             _lib.stream_ptr(y.device)), "w8a8")
+        return y
+
+    ref = parts(x, w)
+    _same([i8.w8a8_linear(x, w)], [ref], "one launch")
+    _same([i8.w8a8_linear(_shifted(x), w)], [ref], "unaligned x")
+    _same([i8.w8a8_linear(x.t().contiguous().t(), w.t().contiguous().t())], [ref], "strided")
+    _same([i8.w8a8_linear(x[None], w)], [ref[None]], "batch")
+    other = torch.bfloat16 if dtype != torch.bfloat16 else torch.float32
+    _same([i8.w8a8_linear(x, w.to(other))], [parts(x, w.to(other))], "two dtypes")
