@@ -492,7 +492,7 @@ extern "C" int64_t sqx_fp8_skinny_workspace_bytes(int64_t m, int64_t rows, int64
   return fp8_ws_bytes(m, rows, cols, SkinnyShape{0, 2, 8, splits > 0 ? splits : 1, false});
 }
 
-// Shared by sqx_fp8_linear (sh from fp8_default_shape unless k_slices > 0) and sqx_fp8_skinny.
+// Shared by sqx_fp8_linear (sh from skinny64_default_shape unless k_slices > 0) and sqx_fp8_skinny.
 static int fp8_linear_impl(const uint8_t* wt, const float* w_scale, const void* x, int act_dtype, void* y, int y_dtype,
                            const void* bias, int64_t m, int64_t rows, int64_t cols, int k_slices, SkinnyShape sh,
                            void* ws, int64_t ws_bytes, sqx_stream_t stream, const char* fn) {
