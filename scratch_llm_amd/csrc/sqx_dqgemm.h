@@ -377,7 +377,9 @@ __global__ __launch_bounds__(2 * TNC * KG, 2) void dq_gemm_kernel(const uint16_t
   if (S >= NS - 1) wait_vmcnt<kPerStage * (Q == 2 ? NS - 2 : NS - 3)>();
   else wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
-  const int Sf = (s0 + S) * 64 > K ? S - 1 : S;  // stages of this split whose columns are all below K
+  // stages of this split whose columns are all below K: 4-bit weights are padded to 128 columns, so at K % 128 of 1..63
+  // the last two stages are not, and the next row's activations must not enter them (0 * Inf is NaN)
+  const int Sf = min(S, K / 64 - s0);
   int s = 0, cur = 0;                            // cur: slot of stage s
   auto wrap = [](int v) { return v >= NS ? v - NS : v; };
   auto phase_end = [&]() {

@@ -105,3 +105,35 @@ def test_gemm_ring_edges_4bit(m, n, k):
     w = f4.dequantize_mxfp4(packed.to(DEV), e8.to(DEV)).double().cpu().numpy()
     y = f4.fp4_linear_tiled(x.to(DEV), f4.tile_mxfp4_packed(packed.to(DEV), e8.to(DEV)))
     _check(y, xd @ w.T, np.abs(xd) @ np.abs(w).T, k, torch.bfloat16, "mxfp4")
+
+
+# k % 128 of 32, 64, 96: the padded last 128 columns leave one or two of the k-stages past k
+@pytest.mark.parametrize("k", [1312, 1344, 1376])
+@pytest.mark.parametrize("m,n", [(300, 8200), (1000, 8200)])  # 128 x 128 and 256 x 256 output tiles
+@pytest.mark.parametrize("fmt", ["int4", "mxfp4"])
+def test_gemm_rows_stay_apart(m, n, k, fmt):
+    """Inf and NaN in the first columns of some rows leave every other row's bits as they were."""
+    from scratch_llm_amd.quant import int4_group as i4
+    from scratch_llm_amd.quant import nvfp4_mxfp4 as f4
+
+    print_case("gemm rows apart", fmt, f"m={m}", f"n={n}", f"k={k}")
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    if fmt == "int4":
+        q = torch.randint(-8, 8, (n, k), generator=g, dtype=torch.int8).to(DEV)
+        tw = i4.tile_int4(q, torch.rand(n, k // 32, generator=g).to(DEV) + 0.5, None, 32)
+        run = i4.int4_linear_tiled
+    else:
+        packed = torch.randint(0, 256, (n, k // 2), generator=g, dtype=torch.uint8).to(DEV)
+        e8 = torch.randint(118, 123, (n, k // 32), generator=g, dtype=torch.uint8).to(DEV)
+        tw, run = f4.tile_mxfp4_packed(packed, e8), f4.fp4_linear_tiled
+    y = run(x, tw)
+    assert bool(torch.isfinite(y).all())
+    bad = torch.tensor([1, 77, m - 1])
+    x[bad, :64:7] = float("inf")
+    x[bad, 3:64:9] = float("nan")
+    z = run(x, tw)
+    keep = torch.ones(m, dtype=torch.bool)
+    keep[bad] = False
+    assert torch.equal(z[keep.to(DEV)], y[keep.to(DEV)])
+    assert bool(torch.isnan(z[bad.to(DEV)]).all())
