@@ -1113,10 +1113,11 @@ extern "C" int sqx_fp4_skinny(const uint8_t* wt, const uint8_t* st, int fmt, con
   if (tiles > 0) sh.R = tiles;
   if (waves > 0) sh.waves = waves;
   if (splits > 0) sh.S = splits;
-  SQX_REQUIRE(m >= 1 && m <= 64 && rows > 0 && cols > 0 && cols % 32 == 0, SQX_E_ARG,
-              "%s: bad shape m=%lld rows=%lld cols=%lld (1..64 rows, cols %% 32 == 0)", fn, (long long)m, (long long)rows,
-              (long long)cols);
   SQX_REQUIRE(fmt == SQX_FP4_MX || fmt == SQX_FP4_NV, SQX_E_ARG, "%s: bad fmt %d", fn, fmt);
+  const int mult = fmt == SQX_FP4_NV ? 16 : 32;  // as sqx_fp4_linear; the kernels mask in steps of 8 columns
+  SQX_REQUIRE(m >= 1 && m <= 64 && rows > 0 && cols > 0 && cols % mult == 0, SQX_E_ARG,
+              "%s: bad shape m=%lld rows=%lld cols=%lld (1..64 rows, cols %% %d == 0)", fn, (long long)m, (long long)rows,
+              (long long)cols, mult);
   SQX_REQUIRE(act_dtype == SQX_DTYPE_BF16 || act_dtype == SQX_DTYPE_F16, SQX_E_ARG, "%s: activations must be BF16 or F16",
               fn);
   SQX_REQUIRE(rows < ((int64_t)1 << 31) && 64 * cols * 2 < ((int64_t)1 << 31), SQX_E_ARG,

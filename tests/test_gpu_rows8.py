@@ -94,3 +94,18 @@ def test_int8_rows(m, n, k):
     # the GEMV (short shapes) sums codes offset by 128 and takes 128 * sum(x) off again
     off = 128.0 * s.double().numpy().T * np.abs(xd).sum(1, keepdims=True)
     _check(y, xd @ wd.T + b, np.abs(xd) @ np.abs(wd).T + np.abs(b) + 2 * off, k, f"int8 {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 40, 16), (8, 10240, 176), (20, 6160, 528), (33, 520, 4112), (63, 16400, 48)])
+def test_nvfp4_rows_of_16_columns(m, n, k):
+    """NVFP4 rows that end in half a 32-column chunk, on the kernels of 2..63 rows."""
+    from scratch_llm_amd.quant import nvfp4_mxfp4 as f4
+
+    print_case("nvfp4 k % 32 == 16", f"m={m}", f"n={n}", f"k={k}")
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    q = f4.nvfp4_quantize(torch.randn(n, k, generator=g).to(DEV) * 0.02)
+    wd = f4.nvfp4_dequantize(q).double().cpu().numpy()
+    y = f4.fp4_linear_tiled(x.to(DEV), f4.tile_fp4(q))
+    xd = x.double().numpy()
+    _check(y, xd @ wd.T, np.abs(xd) @ np.abs(wd).T, k, f"nvfp4 {m}x{n}x{k}")
