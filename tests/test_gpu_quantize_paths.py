@@ -177,3 +177,25 @@ def test_w8a8_one_launch(m, n, k, dtype):
     _same([i8.w8a8_linear(x[None], w)], [ref[None]], "batch")
     other = torch.bfloat16 if dtype != torch.bfloat16 else torch.float32
     _same([i8.w8a8_linear(x, w.to(other))], [parts(x, w.to(other))], "two dtypes")
+
+
+# more rows than a launch holds workgroups of 256 threads: rows too short for a workgroup each
+@pytest.mark.parametrize("cols", [8, 16])
+def test_int8_many_short_rows(cols):
+    from scratch_llm_amd.quant import int8 as i8
+
+    rows = 1 << 24
+    print_case("int8 many short rows", f"{rows}x{cols}")
+    g = torch.Generator(device=DEV).manual_seed(cols)
+    x = torch.randn(rows, cols, device=DEV, generator=g, dtype=torch.bfloat16)
+    parts = [slice(0, 100), slice(rows // 2 - 50, rows // 2 + 50), slice(rows - 100, rows)]
+    for quantize in (i8.quantize_symmetric, i8.quantize_affine):
+        whole = quantize(x, axis=0)
+        for p in parts:
+            _same([t[p] for t in whole], quantize(x[p].contiguous(), axis=0), f"{quantize.__name__} rows {p.start}")
+        del whole
+    if cols % 16 == 0:
+        w = torch.randn(3, cols, device=DEV, generator=g, dtype=torch.bfloat16)
+        y = i8.w8a8_linear(x, w)
+        for p in parts:
+            _same([y[p]], [i8.w8a8_linear(x[p].contiguous(), w)], f"w8a8 rows {p.start}")
