@@ -156,9 +156,18 @@ __global__ __launch_bounds__(256) void fp8_dequantize_kernel(const uint8_t* __re
 }
 
 // Per-head amax over (batch, tokens, head_dim) of x [B, H, inner] (fp8_kv_per_head.py:77-91), then
-// scale = max(amax / 448, MIN_SCALE). Workgroups (slice, head, batch row) reduce a slice of one head each and join
-// through an integer maximum of the fp32 bits, which orders non-negative floats and puts NaN above infinity, so
-// the result does not depend on the order. (One workgroup per head read 117 MB in 7.7 ms; 54 us now.)
+// scale = max(amax / 448, MIN_SCALE). Two forms:
+//  * up to one slice, kHeadSlice elements, a head (a step's or a short prompt's keys), one workgroup per head and one
+//    launch, whose latency is most of such a call: bf16, here and in the form below, 1 x 8 x 128 3.2 and 6.4 us,
+//    64 x 8 x 128 3.8 and 12.1, 1 x 8 x 16384 4.6 and 7.5.
+//  * beyond, workgroups (slice, head, batch row) reduce a slice of one head each and join through an integer maximum
+//    of the fp32 bits, which orders non-negative floats and puts NaN above infinity, so the result does not depend on
+//    the order. (One workgroup per head read 117 MB in 7.7 ms; 54 us so.)
+__device__ inline void finish_head(float am, int64_t h, float* amax, float* scale) {
+  const float q = __fdiv_rn(am, kE4M3Max);
+  if (amax != nullptr) amax[h] = am;
+  if (scale != nullptr) scale[h] = q != q ? q : fmaxf(q, kFp8MinScale);
+}
 constexpr int kHeadSlice = 16384;  // elements of one head a workgroup reads
 __global__ void fp8_head_clear_kernel(uint32_t* __restrict__ bits, int64_t H) {
   const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -185,13 +194,36 @@ __global__ __launch_bounds__(256) void fp8_head_amax_kernel(const void* __restri
   am = block_max_256(am, red);
   if (threadIdx.x == 0) atomicMax(bits + h, __builtin_bit_cast(uint32_t, fabsf(am)));
 }
-__global__ void fp8_head_scale_kernel(const uint32_t* bits, int64_t H, float* amax, float* scale) {
+__global__ void fp8_head_finish_kernel(const uint32_t* bits, int64_t H, float* amax, float* scale) {
   const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= H) return;
-  const float am = __builtin_bit_cast(float, bits[h]);
-  const float q = __fdiv_rn(am, kE4M3Max);
-  if (amax != nullptr) amax[h] = am;
-  if (scale != nullptr) scale[h] = q != q ? q : fmaxf(q, kFp8MinScale);
+  if (h < H) finish_head(__builtin_bit_cast(float, bits[h]), h, amax, scale);
+}
+template <int DT>
+__global__ __launch_bounds__(256) void fp8_head_scale_kernel(const void* __restrict__ x, int B, int64_t H, int inner,
+                                                             int vec, float* __restrict__ amax,
+                                                             float* __restrict__ scale) {
+  __shared__ float red[4];
+  const int64_t h = blockIdx.x;
+  float am = 0.0f;
+  const uint32_t row = inner, n = B * row;
+  if (vec) {  // row % 8 == 0, aligned
+#pragma unroll 2
+    for (uint32_t i = 8 * threadIdx.x; i < n; i += 8 * 256) {
+      const uint32_t b = i / row;
+      float v[8];
+      load8_f32(x, DT, (b * H + h) * row + (i - b * row), v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) am = nan_max(am, fabsf(v[e]));
+    }
+  } else {
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x; i < n; i += 256) {
+      const uint32_t b = i / row;
+      am = nan_max(am, fabsf(load_f<DT>(x, (b * H + h) * row + (i - b * row))));
+    }
+  }
+  am = block_max_256(am, red);
+  if (threadIdx.x == 0) finish_head(am, h, amax, scale);
 }
 
 // quantize_per_head (fp8_kv_per_head.py:93-96): codes = saturating_cast(fp32(x) / scale[h]) for
@@ -398,12 +430,18 @@ extern "C" int sqx_fp8_head_scale(const void* x, int dtype, int64_t B, int64_t H
   SQX_REQUIRE(B >= 0 && H >= 0 && inner >= 0 && H < (int64_t(1) << 31), SQX_E_ARG, "sqx_fp8_head_scale: bad shape");
   if (H == 0) return SQX_OK;
   SQX_REQUIRE((amax || scale) && (x || B * inner == 0), SQX_E_ARG, "sqx_fp8_head_scale: null pointer");
+  hipStream_t st = as_stream(stream);
+  const int vec = inner % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  if (B <= kHeadSlice && inner <= kHeadSlice && B * inner <= kHeadSlice && H < (int64_t(1) << 24)) {
+    SQX_FP8_DT(dtype, fp8_head_scale_kernel, dim3(static_cast<unsigned>(H)), st, x, static_cast<int>(B), H,
+               static_cast<int>(inner), vec, amax, scale);
+    SQX_LAUNCH_CHECK("sqx_fp8_head_scale");
+    return SQX_OK;
+  }
   // the maxima gather in the output itself (scale, or amax when only that is asked for)
   uint32_t* bits = reinterpret_cast<uint32_t*>(scale ? scale : amax);
-  hipStream_t st = as_stream(stream);
   const dim3 hgrid(static_cast<unsigned>(ceil_div(H, 64)));
   hipLaunchKernelGGL(fp8_head_clear_kernel, hgrid, dim3(64), 0, st, bits, H);
-  const int vec = inner % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
   const int64_t slices = ceil_div(inner, kHeadSlice), es = dtype == SQX_DTYPE_F32 ? 4 : 2;
   // grid y and z are 16-bit: heads and batch rows in turns of at most 65535
   for (int64_t b0 = 0; inner > 0 && b0 < B; b0 += 65535)
@@ -413,7 +451,7 @@ extern "C" int sqx_fp8_head_scale(const void* x, int dtype, int64_t B, int64_t H
       const char* xs = static_cast<const char*>(x) + (b0 * H + h0) * inner * es;
       SQX_FP8_DT(dtype, fp8_head_amax_kernel, grid, st, xs, H, inner, vec, bits + h0);
     }
-  hipLaunchKernelGGL(fp8_head_scale_kernel, hgrid, dim3(64), 0, st, bits, H, amax, scale);
+  hipLaunchKernelGGL(fp8_head_finish_kernel, hgrid, dim3(64), 0, st, bits, H, amax, scale);
   SQX_LAUNCH_CHECK("sqx_fp8_head_scale");
   return SQX_OK;
 }

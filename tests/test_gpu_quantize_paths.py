@@ -199,3 +199,26 @@ def test_int8_many_short_rows(cols):
         y = i8.w8a8_linear(x, w)
         for p in parts:
             _same([y[p]], [i8.w8a8_linear(x[p].contiguous(), w)], f"w8a8 rows {p.start}")
+
+
+# the edge between one workgroup per head and the sliced form (16384 elements a head), rows that split it unevenly,
+# and a head count past one block of the finishing kernel
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,h,t,d", [(1, 1, 1, 1), (1, 8, 1, 128), (64, 8, 2, 128), (3, 5, 41, 131), (16383, 1, 1, 1), (1, 70, 129, 128),
+                                     (129, 3, 1, 128), (0, 4, 3, 8)])
+def test_per_head_amax(b, h, t, d, dtype):
+    from scratch_llm_amd.quant import fp8_kv_per_head as kv
+
+    print_case("per-head amax", f"{b}x{h}x{t}x{d}", str(dtype))
+    g = torch.Generator().manual_seed(b + h + t + d)
+    x = torch.randn(b, h, t, d, generator=g).to(dtype)
+    if b:
+        x[-1, -1, -1, -1] = -30.0  # the last element of the last slice
+    ref = x.float().abs().permute(1, 0, 2, 3).reshape(h, -1).max(dim=1).values if b else torch.zeros(h)
+    assert torch.equal(kv.per_head_amax(x.to(DEV)).float().cpu().reshape(-1), ref)
+    want = (ref / 448.0).clamp_min(1.0 / (448.0 * 512.0))
+    assert torch.equal(kv.per_head_scale(x.to(DEV)).float().cpu().reshape(-1), want)
+    if b and h > 1:
+        x[0, 0, 0, 0], x[b // 2, 1, 0, d // 2] = float("nan"), float("inf")
+        a = kv.per_head_amax(x.to(DEV)).float().cpu().reshape(-1)
+        assert bool(torch.isnan(a[0])) and float(a[1]) == float("inf") and torch.equal(a[2:], ref[2:])
