@@ -848,9 +848,33 @@ extern "C" int sqx_int8_linear(const uint8_t* wt, const float* scale, const void
   return SQX_OK;
 }
 
+// The launch for 2..64 rows: FP8's, but for the shapes where the GEMV is the faster one. FP8 quantizes its rows in a
+// launch of its own first and its GEMV has no such head start, so its lines are not int8's. From a sweep of bf16
+// activations at 2..64 rows, 512..28672 weight rows and 512..14336 columns (us, GEMV and row-tiled): 512 -> 512 at
+// m = 17 / 64 4.0 / 6.0 and 7.3 / 9.7; 1536 -> 3000 at m = 33 7.0 and 13.3; 4096 -> 16384 at m = 2 13.4 and 16.0;
+// 4096 -> 4096 at m = 24 / 64 9.9 / 18.2 and 10.0 / 15.3.
+static constexpr GemvUntil kInt8Gemv[] = {
+    { 128, {kG, kG, 24, 24, 20, 24, 20, 10,  8,  7,  4}},
+    { 255, {kG, kG, kG, kG, 22, 24, 20, 16, 16, 16, 11}},
+    { 256, {kG, kG, kG, kG, 22, 24, 20, 12,  8,  8,  6}},
+    { 383, {kG, kG,  0,  0,  0,  0,  0,  8,  6,  6,  6}},
+    { 512, {kG, kG, kG, kG, kG,  5,  4,  3,  2,  2,  0}},
+    { 639, {kG, kG, 10,  3,  3,  3,  5,  3,  3,  3,  3}},
+    { 895, {kG, kG,  5,  4,  4,  4,  4,  3,  3,  4,  3}},
+    {1023, {kG, kG,  3,  3,  3,  3,  2,  2,  0,  2,  2}},
+    {1199, {kG, kG, kG, kG,  5, kG,  7,  5,  3,  3,  2}},
+    {1343, {kG, kG,  4,  4,  2, kG,  4,  4,  3,  3,  2}},
+    {1919, {kG,  5,  2,  2,  2,  3,  2,  2,  2,  2,  0}},
+    {kAllTiles, {kG,  2,  2,  2,  2,  2,  2,  2,  0,  0,  0}}};
+static SkinnyShape int8_default_shape(int64_t m, int64_t rows, int64_t cols) {
+  SkinnyShape sh = skinny64_default_shape(m, rows, cols);
+  if (gemv_ahead(kInt8Gemv, m, rows, cols)) sh.gemv = true;
+  return sh;
+}
+
 extern "C" int64_t sqx_int8_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits) {
   if (m <= 0 || m > 64 || rows <= 0 || cols <= 0) return 0;
-  const SkinnyShape sh = skinny64_default_shape(m, rows, cols);
+  const SkinnyShape sh = int8_default_shape(m, rows, cols);
   const int S = splits > 0 ? splits : sh.gemv ? 1 : sh.S;
   return skinny_workspace_bytes(m, rows, skinny_splits(ceil_div(cols, 64), S));
 }
@@ -860,7 +884,7 @@ extern "C" int sqx_int8_skinny(const uint8_t* wt, const float* scale, const void
                                int splits, void* ws, int64_t ws_bytes, sqx_stream_t stream) {
   const char* fn = "sqx_int8_skinny";
   const bool choose = tiles <= 0 && waves <= 0 && splits <= 0;
-  SkinnyShape sh = skinny64_default_shape(m, rows, cols);
+  SkinnyShape sh = int8_default_shape(m, rows, cols);
   const int64_t KB = ceil_div(cols, 64);
   // the GEMV: the library's choice for the shape, or a row tile group beyond the 32-bit offsets
   if ((choose && sh.gemv) || 4 * KB * 1024 >= ((int64_t)1 << 31))

@@ -737,10 +737,30 @@ inline SkinnyShape skinny_default_shape(int64_t m, int64_t rows, int64_t cols, i
   return s;
 }
 
-// The launch the library picks for m rows of the formats with 64-column blocks (FP8, int8; 16-bit output), from
-// a measured sweep of FP8 at the Llama-3-8B shapes (4096 -> 1024 / 4096 / 6144 / 28672, 14336 -> 4096) at m = 2..64. R tiles of 16 weight rows
-// per workgroup share each activation fragment, `waves` waves split its k-blocks, S workgroups split
-// K; `gemv` marks shapes where the GEMV (one workgroup per tile) is faster:
+// Where the decode GEMV stays ahead of the row-tiled kernels: short rows of weights, whose few k-blocks do not pay for
+// the split and its reduce, and few rows of activations, which cost the GEMV little. For weights of at most `tiles`
+// 16-row tiles: the columns, in units of 512, from which an m-row product leaves the GEMV (kG: never), for m of 2,
+// 3..4, 5, 6, 7..8, 9..11, 12..16, 17..20, 21..32, 33..40 and 41..64.
+struct GemvUntil {
+  int tiles;
+  uint8_t cols512[11];
+};
+constexpr uint8_t kG = 255;
+constexpr int kAllTiles = 1 << 30;
+template <int N>
+inline bool gemv_ahead(const GemvUntil (&table)[N], int64_t m, int64_t rows, int64_t cols) {
+  static constexpr int kLast[11] = {2, 4, 5, 6, 8, 11, 16, 20, 32, 40, 64};  // the last m of each column
+  int c = 0, t = 0;
+  while (c < 10 && m > kLast[c]) ++c;
+  while (t < N - 1 && ceil_div(rows, 16) > table[t].tiles) ++t;
+  const int until = table[t].cols512[c];
+  return until == kG || cols < 512 * (int64_t)until;
+}
+
+// The launch the library picks for m rows of the formats with 64-column blocks (FP8; int8 with its own rule for the
+// GEMV; 16-bit output), from a measured sweep of FP8 at the Llama-3-8B shapes (4096 -> 1024 / 4096 / 6144 / 28672,
+// 14336 -> 4096) at m = 2..64. R tiles of 16 weight rows per workgroup share each activation fragment, `waves` waves
+// split its k-blocks, S workgroups split K; `gemv` marks shapes where the GEMV (one workgroup per tile) is faster:
 //   >= 1024 tiles          R = 2 (m <= 8) or 4, 4 waves, no split;
 //   384 .. 1023 tiles      the GEMV for m <= 4, else R = 2 with 8 waves;
 //   fewer, K >= 8192       the GEMV for m <= 4, else 8 waves and 4 splits, R = 2 (m <= 8) or 4;

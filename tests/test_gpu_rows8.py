@@ -77,8 +77,11 @@ def test_fp4_launch_shapes(m, variant, tiles, waves, splits):
     _check(y, xd @ wd.T, np.abs(xd) @ np.abs(wd).T, k, "fp4 shape")
 
 
+# the GEMV's side of the choice, then the row-tiled kernel's (every range of weight rows that it takes)
 @pytest.mark.parametrize("m,n,k", [(2, 16, 8), (5, 1000, 72), (16, 4096, 4096), (17, 40, 200), (33, 6160, 520), (64, 16400, 136),
-                                   (20, 1024, 8200), (64, 4096, 1032)])
+                                   (20, 1024, 8200), (64, 4096, 1032),
+                                   (16, 1030, 10248), (5, 5200, 8200), (64, 4096, 3080), (36, 3000, 8200), (12, 6160, 2056),
+                                   (8, 10248, 2056), (48, 14330, 1032), (20, 18440, 2568), (4, 28680, 2568), (64, 32776, 72)])
 def test_int8_rows(m, n, k):
     from scratch_llm_amd.quant import int8
 
@@ -109,3 +112,39 @@ def test_nvfp4_rows_of_16_columns(m, n, k):
     y = f4.fp4_linear_tiled(x.to(DEV), f4.tile_fp4(q))
     xd = x.double().numpy()
     _check(y, xd @ wd.T, np.abs(xd) @ np.abs(wd).T, k, f"nvfp4 {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("tiles,waves,splits", [(2, 8, 1), (4, 4, 2), (2, 1, 3), (4, 8, 4), (2, 4, 16)])
+@pytest.mark.parametrize("m", [1, 8, 33, 64])
+def test_int8_launch_shapes(m, tiles, waves, splits):
+    """The row-tiled kernel with an explicit launch shape, partial row tiles and a partial last k-block among them."""
+    from scratch_llm_amd import _lib
+    from scratch_llm_amd.quant import int8
+
+    n, k = 1030, 1432
+    print_case("int8 launch shape", f"m={m}", f"tiles={tiles}", f"waves={waves}", f"splits={splits}")
+    g = torch.Generator().manual_seed(m)
+    q = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    s = torch.rand(n, 1, generator=g) * 1e-3 + 1e-4
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    tw, lib, xg = int8.tile_int8(q.to(DEV), s.to(DEV)), _lib.load(), x.to(DEV)
+    y = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ws = torch.empty(max(int(lib.sqx_int8_skinny_workspace_bytes(m, n, k, splits)) // 4, 1), device=DEV)
+    _lib.check(lib.sqx_int8_skinny(tw.wt.data_ptr(), tw.scale.data_ptr(), xg.data_ptr(), _lib.DTYPE_BF16, y.data_ptr(), None,
+                                   m, n, k, tiles, waves, splits, ws.data_ptr(), ws.numel() * 4, _lib.stream_ptr(xg.device)),
+               "sqx_int8_skinny")
+    xd, wd = x.double().numpy(), q.double().numpy() * s.double().numpy()
+    _check(y, xd @ wd.T, np.abs(xd) @ np.abs(wd).T, k, "int8 shape")
+
+
+def test_few_rows_ask_for_no_workspace():
+    """The GEMV's sizes need none, and a size is asked for once."""
+    from scratch_llm_amd.quant import int8
+
+    q = torch.randint(-128, 128, (512, 512), dtype=torch.int8, device=DEV)
+    tw, x = int8.tile_int8(q, torch.ones(512, 1, device=DEV)), torch.randn(2, 512, device=DEV, dtype=torch.bfloat16)
+    int8.int8_linear_tiled(x, tw)
+    before = int8._rows_workspace.cache_info()
+    int8.int8_linear_tiled(x, tw)
+    after = int8._rows_workspace.cache_info()
+    assert (after.hits, after.misses) == (before.hits + 1, before.misses) and int8._rows_workspace(2, 512, 512) == 0
