@@ -1078,7 +1078,37 @@ extern "C" int sqx_fp4_linear(const uint8_t* wt, const uint8_t* st, int fmt, con
 //                              m = 4 / 32: 38.7 / 110.1 -> 26.7 / 33.7)
 //   640..1023 tiles, shorter K 4 x 8 to 8 rows, LDS-staged 1 x 8 at 17..32 (4096 -> 14336 at m = 4 / 32: 11.0 / 34.2 ->
 //                              9.2 / 13.3)
-static SkinnyShape fp4_default_shape(int64_t m, int64_t rows, int64_t cols, bool have_ws) {
+// and the GEMV where it is the faster kernel, by format (NVFP4's scales make both kernels decode in more steps). From
+// a sweep of bf16 activations at 2..63 rows, 512..128256 weight rows and 512..14336 columns (us, GEMV and row-tiled;
+// MXFP4, NVFP4): 512 -> 512 at m = 17 4.1 and 6.6, 4.4 and 6.7; 1536 -> 3072 at m = 33 7.1 and 9.6, 7.2 and 10.8;
+// 512 -> 28672 at m = 2 4.2 and 5.8, 5.0 and 6.4; 4096 -> 4096 at m = 17 / 32 7.9 / 10.5 and 8.8 / 10.3, 8.1 / 10.6 and
+// 9.0 / 10.4.
+static constexpr GemvUntil kMxGemv[] = {
+    {  64, {kG, kG, kG, kG, kG, 20, 14,  8,  8,  8,  6}},
+    { 256, {kG, kG, kG, kG, 20, 18, 16, 11, 11,  8,  6}},
+    { 383, { 0,  0,  0,  0,  0, 12, 12,  7,  6,  0,  0}},
+    { 512, {kG, 18, 10, 10,  7,  5,  0,  3,  0,  0,  0}},
+    { 639, {24, 20, 10, 10,  7,  3,  3,  3,  2,  0,  0}},
+    { 895, {kG, 18, 10,  8,  6,  5,  4,  0,  0,  0,  0}},
+    {1023, {24,  7,  5,  4,  4,  4,  3,  0,  0,  0,  0}},
+    {1343, {kG, 16, 10,  7,  5,  5,  3,  0,  0,  0,  0}},
+    {1919, { 5,  5,  3,  3,  3,  3,  2,  0,  0,  0,  0}},
+    {3071, { 3,  2,  2,  2,  2,  2,  2,  0,  0,  0,  0}},
+    {kAllTiles, { 2,  2,  0,  0,  0,  0,  0,  0,  0,  0,  0}}};
+static constexpr GemvUntil kNvGemv[] = {
+    {  64, {kG, kG, kG, kG, 24, 18, 16,  8,  8,  8,  8}},
+    { 256, {kG, kG, kG, kG, 22, 22, 16, 11, 11,  8,  8}},
+    { 383, {kG, kG,  0,  0,  0,  0,  0, 11,  8,  3,  2}},
+    { 512, {kG, 20, 10, 10,  5,  5,  2,  3,  2,  3,  2}},
+    { 639, {kG, 20, 10, 10,  7,  3,  3, 10, 10,  0,  0}},
+    { 895, {kG, 24, 24, 10,  7,  5,  5,  2,  1,  0,  0}},
+    {1023, {28, 10,  5,  5,  4,  4,  3,  0,  0,  0,  0}},
+    {1199, {kG, kG, kG, 10,  7,  4,  3,  3,  3,  2,  0}},
+    {1343, {kG, kG, kG, kG,  8,  8,  3,  2,  2,  0,  0}},
+    {1919, {kG,  5,  3,  3,  3,  3,  3,  2,  0,  0,  0}},
+    {3071, { 2,  2,  2,  2,  2,  2,  2,  0,  0,  0,  0}},
+    {kAllTiles, { 2,  2,  0,  0,  0,  0,  0,  0,  0,  0,  0}}};
+static SkinnyShape fp4_row_tiled_shape(int64_t m, int64_t rows, int64_t cols, bool have_ws) {
   const int64_t T = ceil_div(rows, 16), KB = ceil_div(cols, 128);
   if (m >= 2 && T >= 1024 && T < 4096 && m <= 8) return SkinnyShape{0, 4, 4, 1, false};
   if (m >= 2 && T >= 384 && T < 1024 && KB >= 64 && have_ws)
@@ -1090,11 +1120,21 @@ static SkinnyShape fp4_default_shape(int64_t m, int64_t rows, int64_t cols, bool
   return sh;
 }
 
+static SkinnyShape fp4_default_shape(int fmt, int64_t m, int64_t rows, int64_t cols, bool have_ws) {
+  SkinnyShape sh = fp4_row_tiled_shape(m, rows, cols, have_ws);
+  if (fmt == SQX_FP4_NV ? gemv_ahead(kNvGemv, m, rows, cols) : gemv_ahead(kMxGemv, m, rows, cols)) sh.gemv = true;
+  return sh;
+}
+
 extern "C" int64_t sqx_fp4_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits) {
   if (m <= 0 || m > 64 || rows <= 0 || cols <= 0) return 0;
-  const SkinnyShape sh = fp4_default_shape(m, rows, cols, true);
-  const int S = splits > 0 ? splits : sh.gemv ? 1 : sh.S;
-  return skinny_workspace_bytes(m, rows, skinny_splits(ceil_div(cols, 128), S));
+  int64_t need = 0;  // of either format
+  for (int fmt : {SQX_FP4_MX, SQX_FP4_NV}) {
+    const SkinnyShape sh = fp4_default_shape(fmt, m, rows, cols, true);
+    const int S = splits > 0 ? splits : sh.gemv ? 1 : sh.S;
+    need = std::max(need, skinny_workspace_bytes(m, rows, skinny_splits(ceil_div(cols, 128), S)));
+  }
+  return need;
 }
 
 extern "C" int sqx_fp4_skinny(const uint8_t* wt, const uint8_t* st, int fmt, const float* s_global, const void* x,
@@ -1102,7 +1142,7 @@ extern "C" int sqx_fp4_skinny(const uint8_t* wt, const uint8_t* st, int fmt, con
                               int variant, int tiles, int waves, int splits, void* ws, int64_t ws_bytes,
                               sqx_stream_t stream) {
   const char* fn = "sqx_fp4_skinny";
-  SkinnyShape sh = fp4_default_shape(m, rows, cols, ws != nullptr);
+  SkinnyShape sh = fp4_default_shape(fmt, m, rows, cols, ws != nullptr);
   const int64_t KB = ceil_div(cols, 128);
   // the GEMV: the library's choice for the shape, or a weight beyond the 32-bit offsets of a workgroup's tiles
   if ((variant < 0 && tiles <= 0 && waves <= 0 && splits <= 0 && sh.gemv) || 4 * KB * 1024 >= ((int64_t)1 << 31))

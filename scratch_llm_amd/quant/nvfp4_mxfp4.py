@@ -16,6 +16,8 @@ dequantized activation rows instead (:func:`mxfp4_fake_quant_rows`, exact in bf1
 
 from __future__ import annotations
 
+import functools
+
 import torch
 from torch import Tensor
 
@@ -327,6 +329,13 @@ def e4m3_values(codes: Tensor) -> Tensor:
     return out.reshape(codes.shape)
 
 
+@functools.lru_cache(maxsize=4096)
+def _rows_workspace(m: int, rows: int, cols: int) -> int:
+    """Workspace bytes of 2..``GEMM_MIN_M - 1`` rows (0 where the GEMV is chosen), asked of the library once per size:
+    at a few rows another native call per linear shows."""
+    return int(_lib.load().sqx_fp4_skinny_workspace_bytes(m, rows, cols, 0))
+
+
 def fp4_linear_tiled(x: Tensor, tw: FP4Tiled, bias: Tensor | None = None, out_dtype: torch.dtype | None = None,
                      k_slices: int | None = None) -> Tensor:
     """``x @ W.T (+ bias)`` for a tiled FP4 weight. ``x`` is ``[..., cols]``: bf16 / fp16 run as they
@@ -378,7 +387,7 @@ def fp4_linear_tiled(x: Tensor, tw: FP4Tiled, bias: Tensor | None = None, out_dt
                                         _lib.sqx_dtype(x.dtype), y.data_ptr(), ydt, _lib.ptr(b), m, tw.rows, tw.cols,
                                         *_lib.ws_args(ws), s), "fp4_linear")
         elif 2 <= m < GEMM_MIN_M and k_slices is None and not yf32:
-            nb = int(lib.sqx_fp4_skinny_workspace_bytes(m, tw.rows, tw.cols, 0))
+            nb = _rows_workspace(m, tw.rows, tw.cols)
             ws = torch.empty(nb // 4, dtype=torch.float32, device=dev) if nb > 0 else None
             _lib.check(lib.sqx_fp4_skinny(tw.wt.data_ptr(), tw.st.data_ptr(), tw.fmt, _lib.ptr(tw.s_global), x2.data_ptr(),
                                           _lib.sqx_dtype(x.dtype), y.data_ptr(), _lib.ptr(b), m, tw.rows, tw.cols, -1, 0,

@@ -29,7 +29,10 @@ def _check(y, ref, mag, k, what):
 
 # partial row tiles, a partial last k-block, fewer k-blocks than waves, every dispatch range of rows
 LINEAR = [(2, 16, 32), (3, 1000, 96), (8, 40, 224), (9, 6150, 512), (16, 4096, 1056), (17, 10240, 160), (32, 16400, 320),
-          (33, 520, 4096), (63, 1024, 8224), (24, 6400, 8192)]
+          (33, 520, 4096), (63, 1024, 8224), (24, 6400, 8192),
+          # the row-tiled kernels' side of the choice, for either format
+          (6, 28700, 1568), (9, 6150, 2592), (12, 4096, 9248), (4, 10250, 12320), (18, 14400, 544), (40, 28700, 1056),
+          (13, 18000, 2080), (2, 30000, 2592), (36, 5200, 1568), (5, 65552, 96)]
 
 
 @pytest.mark.parametrize("fmt", ["mx", "nv"])
