@@ -602,8 +602,9 @@ __global__ __launch_bounds__(256 * KG) void skinny_lds_kernel(const typename W::
 }
 
 // y[m, n] = act(sum over s in order of part[s][m][n] (* rs[m] when given) (* cs[n]) (* *gs) + bias[n]);
-// four outputs per thread.
-template <class A>
+// four outputs per thread. SCALED false: a policy without such factors (int4, whose scales are in the sums): its reduce
+// is a launch of a few microseconds that the three tests per output lengthen by 0.1.
+template <class A, bool SCALED>
 __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restrict__ part, int S, int M, int N,
                                                             const uint16_t* __restrict__ bias,
                                                             uint16_t* __restrict__ y, const float* __restrict__ rs,
@@ -622,12 +623,14 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
       for (int j = 0; j < 4; ++j) v[j] += q[j];
     }
     const int n = static_cast<int>(i % N);
-    const float r = rs ? rs[i / N] : 1.0f, g = gs ? *gs : 1.0f;
+    if constexpr (SCALED) {
+      const float r = rs ? rs[i / N] : 1.0f, g = gs ? *gs : 1.0f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (rs) v[j] *= r;
-      if (cs) v[j] *= cs[n + j];
-      if (gs) v[j] *= g;
+      for (int j = 0; j < 4; ++j) {
+        if (rs) v[j] *= r;
+        if (cs) v[j] *= cs[n + j];
+        if (gs) v[j] *= g;
+      }
     }
     uint32_t lo, hi;
     float o[4];
@@ -640,9 +643,11 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
     for (int64_t e = i; e < i + 4 && e < total; ++e) {
       float v = part[e];
       for (int s = 1; s < S; ++s) v += part[(int64_t)s * total + e];
-      if (rs) v *= rs[e / N];
-      if (cs) v *= cs[e % N];
-      if (gs) v *= *gs;
+      if constexpr (SCALED) {
+        if (rs) v *= rs[e / N];
+        if (cs) v *= cs[e % N];
+        if (gs) v *= *gs;
+      }
       if (bias) v += A::to_f32(bias[e % N]);
       y[e] = A::from_f32(v);
     }
@@ -800,6 +805,9 @@ const float* global_scale(const typename W::Args& wa) {
   else return nullptr;
 }
 
+template <class W>
+inline constexpr bool scaled_reduce = has_row_scale<W>::value || has_out_scales<W>::value || has_global_scale<W>::value;
+
 // The LDS-staged variant: R (1, 2 or 4) tiles per wave, 4 waves per workgroup, S splits along K.
 template <class A, class W>
 hipError_t skinny_lds_launch(const typename W::Args& wa, const uint16_t* x, uint16_t* y, const uint16_t* bias,
@@ -859,8 +867,8 @@ hipError_t skinny_lds_launch(const typename W::Args& wa, const uint16_t* x, uint
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !split || !reduce) return e;
   const int64_t quads = ceil_div(m * rows, 4);
-  hipLaunchKernelGGL(skinny_reduce_kernel<A>, dim3(static_cast<unsigned>(ceil_div(quads, 256))), dim3(256), 0, stream,
-                     ws, S, M, N, bias, y, nullptr, nullptr, global_scale<W>(wa));
+  hipLaunchKernelGGL((skinny_reduce_kernel<A, scaled_reduce<W>>), dim3(static_cast<unsigned>(ceil_div(quads, 256))),
+                     dim3(256), 0, stream, ws, S, M, N, bias, y, nullptr, nullptr, global_scale<W>(wa));
   return hipGetLastError();
 }
 
@@ -925,8 +933,8 @@ hipError_t skinny_launch(const typename W::Args& wa, const uint16_t* x, uint16_t
   const float* cs = nullptr;
   if constexpr (has_row_scale<W>::value) rs = W::row_scales(wa);
   if constexpr (has_out_scales<W>::value) cs = W::out_scales(wa);
-  hipLaunchKernelGGL(skinny_reduce_kernel<A>, dim3(static_cast<unsigned>(ceil_div(quads, 256))), dim3(256), 0, stream,
-                     ws, S, M, N, bias, y, rs, cs, global_scale<W>(wa));
+  hipLaunchKernelGGL((skinny_reduce_kernel<A, scaled_reduce<W>>), dim3(static_cast<unsigned>(ceil_div(quads, 256))),
+                     dim3(256), 0, stream, ws, S, M, N, bias, y, rs, cs, global_scale<W>(wa));
   return hipGetLastError();
 }
 
