@@ -595,8 +595,8 @@ int sqx_int8_skinny(const uint8_t* wt, const float* scale, const void* x, int ac
 /* The same product from 65 rows on (prefill): the dequant GEMM on the tiled int8 weight, whose codes are
  * exact in the activation dtype, with the per-row scale on the fp32 sum. cols % 8 == 0; ws: at least
  * sqx_int8_gemm_workspace_bytes(m, rows, cols) bytes, 16-byte aligned, for the fp32 partials of the K splits
- * (smaller or NULL: one pass per output tile). The query returns -1 for shapes the GEMM does not take
- * (m == 0, operands of 2 GiB and more); sqx_int8_linear takes those. */
+ * (smaller or NULL: one pass per output tile). The query returns -1 for shapes that sqx_int8_linear takes: those
+ * beyond the GEMM (m == 0, operands of 2 GiB and more) and small ones, where it is the faster kernel. */
 int64_t sqx_int8_gemm_workspace_bytes(int64_t m, int64_t rows, int64_t cols);
 int sqx_int8_gemm(const uint8_t* wt, const float* scale, const void* x, int act_dtype, void* y, const void* bias,
                   int64_t m, int64_t rows, int64_t cols, void* ws, int64_t ws_bytes, sqx_stream_t stream);

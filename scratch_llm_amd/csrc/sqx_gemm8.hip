@@ -29,8 +29,15 @@ hipError_t fp8_gemm(const uint8_t* wt, const float* w_scale, const float* x_scal
 
 using namespace sqx;
 
+// Where the GEMV's two passes over a small weight are faster than the GEMM's prologue and its few workgroups (us, GEMV
+// and GEMM: 512 -> 512 at m = 65 / 96 / 128 7.9 / 9.2 / 10.9 and 10.6 / 10.8 / 11.0, 1024 -> 1024 at 65 / 100 9.0 / 11.5
+// and 11.0 / 11.7, 1536 -> 3000 at 72 / 96 12.4 / 14.5 and 13.3 / 14.3, 2048 -> 2000 at 65 13.1 and 12.4).
+static bool int8_gemv_ahead(int64_t m, int64_t rows, int64_t cols) {
+  return (m <= 104 && rows <= 1024 && cols <= 1024) || (m <= 80 && rows <= 3072 && cols <= 1536);
+}
+
 extern "C" int64_t sqx_int8_gemm_workspace_bytes(int64_t m, int64_t rows, int64_t cols) {
-  if (!gemm8_fits(m, rows, cols)) return -1;
+  if (!gemm8_fits(m, rows, cols) || int8_gemv_ahead(m, rows, cols)) return -1;
   return dq_workspace_bytes(dq_plan(m, rows, ceil_div(cols, 64), kDqI8), m, rows);
 }
 

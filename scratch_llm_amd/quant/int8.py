@@ -293,10 +293,17 @@ def _rows_workspace(m: int, rows: int, cols: int) -> int:
     return int(_lib.load().sqx_int8_skinny_workspace_bytes(m, rows, cols, 0))
 
 
+@functools.lru_cache(maxsize=4096)
+def _gemm_workspace(m: int, rows: int, cols: int) -> int:
+    """Workspace bytes of the prefill GEMM, -1 where the decode GEMV takes the shape."""
+    return int(_lib.load().sqx_int8_gemm_workspace_bytes(m, rows, cols))
+
+
 def int8_linear_tiled(x: Tensor, tw: Int8Tiled, bias: Tensor | None = None, k_slices: int | None = None) -> Tensor:
     """``x @ (q * s).T (+ bias)`` for a tiled int8 weight; ``x`` bf16 / fp16 ``[..., in]``. One row,
     or any with ``k_slices`` set, on the streaming decode GEMV; 2..``GEMM_MIN_M - 1`` rows on the library's
-    choice of the GEMV and the row-tiled kernel; from there on the prefill GEMM."""
+    choice of the GEMV and the row-tiled kernel; from there on the prefill GEMM (small weights: the GEMV
+    for some rows more)."""
     *batch, k = x.shape
     if k != tw.cols:
         raise ValueError(f"x has in_features={k}, weight expects {tw.cols}")
@@ -310,7 +317,7 @@ def int8_linear_tiled(x: Tensor, tw: Int8Tiled, bias: Tensor | None = None, k_sl
     y = torch.empty(m, tw.rows, dtype=x.dtype, device=dev)
     b = None if bias is None else bias.to(x.dtype).contiguous()
     lib = _lib.load()
-    nb = int(lib.sqx_int8_gemm_workspace_bytes(m, tw.rows, k)) if m >= GEMM_MIN_M and k_slices is None else -1
+    nb = _gemm_workspace(m, tw.rows, k) if m >= GEMM_MIN_M and k_slices is None else -1
     with torch.cuda.device(dev):
         if nb >= 0:
             ws = torch.empty(nb // 4, dtype=torch.float32, device=dev) if nb > 0 else None

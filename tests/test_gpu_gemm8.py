@@ -61,7 +61,7 @@ def test_int8_gemm(m, n, k, dtype):
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("m,n,k", SHAPES + [(70, 1024, 1024), (71, 1024, 1024)])  # the GEMV's last rows, the GEMM's first
 def test_fp8_gemm(m, n, k, out_dtype):
     from scratch_llm_amd.quant import fp8_weights as f8
 
