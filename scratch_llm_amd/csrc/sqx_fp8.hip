@@ -373,10 +373,13 @@ static bool fp8_float_dtype(int d) { return d == SQX_DTYPE_F32 || d == SQX_DTYPE
 
 // Per-row quantize into codes (optional) and bf16 values (optional): the register kernel for aligned rows with
 // cols % 8 == 0 and cols <= 32768, else the generic one. 1024 threads a row when there are few rows (latency),
-// 256 from 512 rows on, where the rows fill the chip.
+// 256 from 512 rows on, where the rows fill the chip. fp32 rows, which the generic kernel reads 4 bytes a lane, take
+// the register kernel from 128 columns on and 256 threads to 2048 (generic and register kernel: 300000 x 16 180 and
+// 196 us, 262144 x 64 158 and 172; 1 x 128 with 1024 threads 3.1 and 3.3).
 static void fp8_quantize_rows_launch(const void* x, int dtype, int64_t rows, int64_t cols, uint8_t* codes, float* scale,
                                      uint16_t* vals, hipStream_t s) {
-  const bool vec = cols % 8 == 0 && cols <= 32768 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+  const bool vec = cols % 8 == 0 && cols >= (dtype == SQX_DTYPE_F32 ? 128 : 8) && cols <= 32768 &&
+                   reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                    (codes == nullptr || reinterpret_cast<uintptr_t>(codes) % 8 == 0) &&
                    (vals == nullptr || reinterpret_cast<uintptr_t>(vals) % 16 == 0);
   if (vec) {
@@ -384,7 +387,7 @@ static void fp8_quantize_rows_launch(const void* x, int dtype, int64_t rows, int
 #define SQX_Q8(DT_, N_, NT_) \
   hipLaunchKernelGGL((fp8_quantize_rows8_kernel<DT_, N_, NT_>), grid, dim3(NT_), 0, s, x, cols, codes, scale, vals)
 #define SQX_Q8N(DT_)                                       \
-  if (rows >= 512 && cols <= 2048) SQX_Q8(DT_, 1, 256);      \
+  if (cols <= 2048 && (rows >= 512 || DT_ == SQX_DTYPE_F32)) SQX_Q8(DT_, 1, 256); \
   else if (rows >= 512 && cols <= 4096) SQX_Q8(DT_, 2, 256); \
   else if (rows >= 512 && cols <= 8192) SQX_Q8(DT_, 4, 256); \
   else if (rows >= 512 && cols <= 16384) SQX_Q8(DT_, 8, 256); \
