@@ -563,7 +563,7 @@ int sqx_int8_dequantize_affine(const uint8_t* q, int64_t A, int64_t B, int64_t C
 int sqx_w8a8_gemm(const int8_t* qx, const void* sx, int sx_dtype, const int8_t* qw, const void* sw,
                   int sw_dtype, float* y, int64_t m, int64_t n, int64_t k, sqx_stream_t stream);
 /* The whole of w8a8_linear for x [m, k] and w [n, k] of one dtype, both 16-byte aligned, k % 16 == 0, k <= 32768,
- * m + n < 2**24 and, for k < 128, m + n <= 2048: the rows of both quantized (int8.py:102-125) in one launch, then
+ * m + n < 2**24 and, for k < 64, m + n <= 2048: the rows of both quantized (int8.py:102-125) in one launch, then
  * the product. ws: sqx_w8a8_workspace_bytes(m, n, k) bytes (-1: a shape this call does not take), 16-byte aligned. */
 int64_t sqx_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int sqx_w8a8_linear(const void* x, const void* w, int dtype, float eps, float* y, int64_t m, int64_t n, int64_t k,

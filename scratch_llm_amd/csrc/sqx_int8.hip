@@ -619,12 +619,13 @@ static int int8_stats(const void* x, int dtype, int64_t A, int64_t B, int64_t C,
 extern "C" int64_t sqx_int8_workspace_bytes(void) { return (int64_t)kStatParts * 8; }
 
 // One pass over the B rows of x (from row B1 on: of x2), for rows of whole 8-element chunks that fit a workgroup's
-// registers. A workgroup a row pays from 128 columns on, and for as few rows as the chip holds workgroups at once:
-// more rows that are shorter leave most lanes idle (bf16, one pass against two: 300000 x 16 230 and 22 us, 65536 x 32
-// 51 and 49; 4096 x 128 6.3 and 7.8, 1000 x 24 4.2 and 6.4). A launch holds fewer than 2**32 threads.
+// registers. A workgroup a row pays from 64 columns on (the affine form, with its two statistics, from 128), and for
+// as few rows as the chip holds workgroups at once: more rows that are shorter leave most lanes idle (bf16, one pass
+// against two: 300000 x 16 230 and 22 us, 65536 x 32 51 and 49, 262144 x 64 201 and 215, affine 275 and 261;
+// 1000 x 24 4.2 and 6.4). A launch holds fewer than 2**32 threads.
 constexpr int64_t kQuantRowsMaxC = 16 * 2048;
-static bool quantize_rows_fits(int64_t B, int64_t C) {
-  return C % 8 == 0 && C <= kQuantRowsMaxC && B < ((int64_t)1 << 24) && (C >= 128 || B <= 2048);
+static bool quantize_rows_fits(int64_t B, int64_t C, bool affine) {
+  return C % 8 == 0 && C <= kQuantRowsMaxC && B < ((int64_t)1 << 24) && (C >= (affine ? 128 : 64) || B <= 2048);
 }
 template <int OP>
 static void launch_quantize_rows(const void* x, const void* x2, int64_t B1, int64_t B, int dtype, int64_t C, float eps,
@@ -656,7 +657,7 @@ static int int8_quantize(const void* x, int dtype, int64_t A, int64_t B, int64_t
   SQX_REQUIRE(x && q && s && (OP == 0 || z), SQX_E_ARG, "%s: null pointer", fn);
   SQX_REQUIRE(B == 1 || B < ((int64_t)1 << 31), SQX_E_ARG, "%s: kept axis too long", fn);
   hipStream_t st = as_stream(stream);
-  if (A == 1 && B > 1 && quantize_rows_fits(B, C) && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+  if (A == 1 && B > 1 && quantize_rows_fits(B, C, OP == 1) && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 8 == 0) {
     launch_quantize_rows<OP>(x, nullptr, B, B, dtype, C, eps, q, s, z, st);
     SQX_LAUNCH_CHECK(fn);
@@ -766,7 +767,7 @@ extern "C" int sqx_w8a8_gemm(const int8_t* qx, const void* sx, int sx_dtype, con
 
 extern "C" int64_t sqx_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   // int8 rows of x, then of w, then their scales (at most fp32)
-  return k > 0 && k % 16 == 0 && m > 0 && n > 0 && quantize_rows_fits(m + n, k) && m * k < ((int64_t)1 << 31) &&
+  return k > 0 && k % 16 == 0 && m > 0 && n > 0 && quantize_rows_fits(m + n, k, false) && m * k < ((int64_t)1 << 31) &&
                  n * k < ((int64_t)1 << 31)
              ? (m + n) * (k + 4)
              : -1;
