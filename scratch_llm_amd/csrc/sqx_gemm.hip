@@ -443,26 +443,31 @@ extern "C" int sqx_mxfp4_gemm_ws(const uint8_t* xt, const uint8_t* xst, const ui
                 as_stream(stream));
 }
 
-// Output tile and K splits of the dequant GEMM, the cheapest under a cost model fitted to a sweep of 65..2048
-// rows at the Llama-3-8B shapes (int8, MXFP4, symmetric and asymmetric int4; every tile with every split).
-// A workgroup fills a CU (its stages take 110 to 150 KiB of LDS), so tiles * S workgroups run in
-// ceil(tiles * S / 256) rounds of ceil(stages / S) stages, plus about 4 us of launch, prologue and epilogue.
-// A stage takes, with a share b of the CUs busy (us):
-//                8-bit           FP4             int4
-//   256 x 256    0.85 + 0.70 b   0.97 + 0.45 b   1.45 + 0.40 b   the fewest bytes and decodes per MFMA
-//   128 x 256    0.68 + 0.30 b   0.70 + 0.18 b   0.95 + 0.30 b
-//   128 x 128    0.47 + 0.12 b   0.57 + 0.03 b   0.67 + 0.06 b   short m or narrow n
-// (int8 4096 -> 4096 at 1000 rows: 42 us on 128 x 128 tiles, 55 us on 256 x 256 in four splits). K splits add
-// 3 us for the reduce launch and 8 bytes per output and split at about 5 TB/s.
+// Output tile and K splits of the dequant GEMM, the cheapest under a cost model fitted to a sweep of 65..2048 rows by
+// 512..28672 weight rows by 512..14336 columns (22 row counts at 22 weights; every tile with every split, int8, MXFP4,
+// NVFP4, symmetric and asymmetric int4). A workgroup fills a CU (its stages take 130 to 160 KiB of LDS; the 8-bit
+// 128 x 256 ring the whole 160), so tiles * S workgroups run in ceil(tiles * S / 256) rounds, each a fixed time
+// (prologue, pipeline fill, epilogue) and ceil(stages / S) stages, which take longer the more CUs are busy. In us,
+// fixed; a stage with one CU busy + what all CUs busy add:
+//                8-bit               MXFP4               NVFP4               int4
+//   256 x 256    3.0; 1.20 + 0.01    3.9; 1.12 + 0.02    3.7; 1.43 + 0.01    3.7; 1.66 + 0.01   fewest bytes and decodes
+//   128 x 256    3.8; 0.68 + 0.11    2.8; 0.72           3.2; 1.07 + 0.05    5.2; 1.08 + 0.01
+//   128 x 128    3.6; 0.40 + 0.08    1.6; 0.48 + 0.08    3.0; 0.65 + 0.09    4.7; 0.58 + 0.11   short m or narrow n
+// A launch takes 4.4 us more, and K splits 3 for the reduce and 1.35 per million outputs and split. The choice is
+// within 0.6 % of the best one over the sweep on average. Without the fixed time, and with MXFP4's stages for
+// NVFP4, wide weights with short rows and NVFP4 went to tiles that are too small: int4 512 -> 28672 at 640 rows 54 us on
+// 128 x 128, 42 on 256 x 256; NVFP4 4096 -> 6144 at 768 rows 77 us on 128 x 256, 61 on 256 x 256 in three splits. The
+// 8-bit column is fitted to int8 and FP8 together (their codes decode in as many steps).
 DqPlan sqx::dq_plan(int64_t m, int64_t rows, int64_t stages, int fmt) {
   struct Tile {
     int tm, tn;
-    double idle[3], busy[3];
+    double fixed[4], stage[4], busy[4];
   };
-  static constexpr Tile kTiles[] = {{256, 256, {0.85, 0.97, 1.45}, {0.70, 0.45, 0.40}},
-                                    {128, 256, {0.68, 0.70, 0.95}, {0.30, 0.18, 0.30}},
-                                    {128, 128, {0.47, 0.57, 0.67}, {0.12, 0.03, 0.06}}};
-  const int f = fmt == kDqInt4 ? 2 : fmt == kDqMx || fmt == kDqNv ? 1 : 0;
+  static constexpr Tile kTiles[] = {
+      {256, 256, {3.0, 3.9, 3.7, 3.7}, {1.20, 1.12, 1.43, 1.66}, {0.01, 0.02, 0.01, 0.01}},
+      {128, 256, {3.8, 2.8, 3.2, 5.2}, {0.68, 0.72, 1.07, 1.08}, {0.11, 0.00, 0.05, 0.01}},
+      {128, 128, {3.6, 1.6, 3.0, 4.7}, {0.40, 0.48, 0.65, 0.58}, {0.08, 0.08, 0.09, 0.11}}};
+  const int f = fmt == kDqInt4 ? 3 : fmt == kDqNv ? 2 : fmt == kDqMx ? 1 : 0;
   DqPlan best{256, 256, 1};
   double best_us = 0.0;
   bool first = true;
@@ -472,8 +477,8 @@ DqPlan sqx::dq_plan(int64_t m, int64_t rows, int64_t stages, int fmt) {
       const int64_t per = ceil_div(stages, S), wgs = tiles * S;
       if (ceil_div(stages, per) != S) continue;  // the last split would be empty
       const double b = wgs >= 256 ? 1.0 : (double)wgs / 256.0;
-      double us = 4.0 + (double)ceil_div(wgs, 256) * (double)per * (t.idle[f] + t.busy[f] * b);
-      if (S > 1) us += 3.0 + (double)S * (double)m * (double)rows * 8.0 / 5e6;
+      double us = 4.4 + (double)ceil_div(wgs, 256) * (t.fixed[f] + (double)per * (t.stage[f] + t.busy[f] * b));
+      if (S > 1) us += 3.0 + (double)S * (double)m * (double)rows * 1.35e-6;
       if (first || us < best_us) best = DqPlan{t.tm, t.tn, S}, best_us = us, first = false;
     }
   }
@@ -498,9 +503,10 @@ int dq_check(const char* fn, const void* x, const void* wt, const void* y, int64
 
 extern "C" int64_t sqx_gemm_workspace_bytes(int64_t m, int64_t rows, int64_t cols) {
   if (m <= 0 || rows <= 0 || cols <= 0) return 0;
-  const int64_t stages = 2 * ceil_div(cols, 128);  // int4 and FP4 plans differ: room for either
-  return std::max(dq_workspace_bytes(dq_plan(m, rows, stages, kDqInt4), m, rows),
-                  dq_workspace_bytes(dq_plan(m, rows, stages, kDqMx), m, rows));
+  const int64_t stages = 2 * ceil_div(cols, 128);  // the 4-bit formats' plans differ: room for each
+  int64_t need = 0;
+  for (int fmt : {kDqInt4, kDqMx, kDqNv}) need = std::max(need, dq_workspace_bytes(dq_plan(m, rows, stages, fmt), m, rows));
+  return need;
 }
 
 extern "C" int sqx_int4_gemm(const uint8_t* wt, const void* st, const void* zt, int param_dtype, const void* x,
