@@ -497,6 +497,10 @@ int sqx_int4_gemm(const uint8_t* wt, const void* st, const void* zt, int param_d
  * the workspace, added in a fixed order by a second kernel (deterministic). 0 = no split. A NULL or
  * smaller workspace runs without the split (same result, slower for small m). */
 int64_t sqx_gemm_workspace_bytes(int64_t m, int64_t rows, int64_t cols);
+/* The output tile (rows of x by rows of the weight) and the K splits that the dequant GEMM takes for a shape when the
+ * workspace has room for them. weight: SQX_GEMM_*. */
+enum { SQX_GEMM_INT4 = 0, SQX_GEMM_MXFP4 = 1, SQX_GEMM_NVFP4 = 2, SQX_GEMM_INT8 = 3, SQX_GEMM_FP8 = 4 };
+int sqx_gemm_plan(int weight, int64_t m, int64_t rows, int64_t cols, int* tile_m, int* tile_n, int* splits);
 
 /* W4A16 linear with fp32 activations (w4a16_linear, int4_group.py:157-164, and awq_linear,
  * awq.py:184-192, which accept any x.dtype and then run F.linear in fp32): x [m, cols] fp32,

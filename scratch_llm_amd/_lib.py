@@ -26,6 +26,7 @@ FP4_SCALE_MX_F32 = 0
 FP4_SCALE_MX_E8M0 = 1
 FP4_SCALE_NV_F32 = 2
 FP4_SCALE_NV_E4M3 = 3
+GEMM_WEIGHTS = ("int4", "mxfp4", "nvfp4", "int8", "fp8")  # SQX_GEMM_* by index
 
 _TORCH_TO_SQX = {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16}
 
@@ -115,6 +116,7 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "sqx_mxfp4_gemm_ws": (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_p, _c_i64,
                                  _c_p]),
     "sqx_gemm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "sqx_gemm_plan": (_c_i, [_c_i, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p]),
     "sqx_int4_gemm": (
         _c_i,
         [_c_p, _c_p, _c_p, _c_i, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p],

@@ -509,6 +509,18 @@ extern "C" int64_t sqx_gemm_workspace_bytes(int64_t m, int64_t rows, int64_t col
   return need;
 }
 
+extern "C" int sqx_gemm_plan(int weight, int64_t m, int64_t rows, int64_t cols, int* tile_m, int* tile_n, int* splits) {
+  static_assert(SQX_GEMM_INT4 == kDqInt4 && SQX_GEMM_MXFP4 == kDqMx && SQX_GEMM_NVFP4 == kDqNv && SQX_GEMM_INT8 == kDqI8 &&
+                SQX_GEMM_FP8 == kDqF8, "one numbering");
+  SQX_REQUIRE(weight >= SQX_GEMM_INT4 && weight <= SQX_GEMM_FP8 && m > 0 && rows > 0 && cols > 0, SQX_E_ARG,
+              "sqx_gemm_plan: bad weight %d or shape", weight);
+  SQX_REQUIRE(tile_m && tile_n && splits, SQX_E_ARG, "sqx_gemm_plan: null pointer");
+  const bool b8 = weight == SQX_GEMM_INT8 || weight == SQX_GEMM_FP8;
+  const DqPlan p = dq_plan(m, rows, b8 ? ceil_div(cols, 64) : 2 * ceil_div(cols, 128), weight);
+  *tile_m = p.tm, *tile_n = p.tn, *splits = p.splits;
+  return SQX_OK;
+}
+
 extern "C" int sqx_int4_gemm(const uint8_t* wt, const void* st, const void* zt, int param_dtype, const void* x,
                              int act_dtype, void* y, const void* bias, int64_t m, int64_t rows, int64_t cols,
                              int64_t group, void* ws, int64_t ws_bytes, sqx_stream_t stream) {

@@ -1,5 +1,5 @@
-"""The dequant GEMM on 8-bit weights (sqx_int8_gemm and sqx_fp8_linear from 65 rows) and the tile, split and
-ring edges of its pipeline for every weight format, on the MI355X.
+"""The dequant GEMM on 8-bit weights (sqx_int8_gemm and sqx_fp8_linear from 65 rows) and the split and ring edges of its
+pipeline, at shapes that mostly take its 128 x 128 tile, on the MI355X (test_gpu_gemm_tiles.py has every tile).
 
 int8 and E4M3 codes are exact in the activation dtype, so int8 differs from the float64 product only by the
 fp32 accumulation, ``(k/32 + 8) * 2**-24 * sum|x w|`` (one rounded 32-term MFMA partial per step, two
@@ -56,7 +56,7 @@ def test_int8_gemm(m, n, k, dtype):
         b = bias.double().numpy()
         ref, mag = ref + b, mag + np.abs(b)
     _check(y, ref, mag, k, dtype, f"int8 {m}x{n}x{k}")
-    # one call's bits do not depend on the rows around them (same plan), and repeat
+    # a second call gives the same bits
     assert torch.equal(y, int8.int8_linear_tiled(x.to(DEV), tw, None if bias is None else bias.to(DEV)))
 
 
@@ -86,7 +86,7 @@ def test_fp8_gemm(m, n, k, out_dtype):
 @pytest.mark.parametrize("k", [128, 256, 384, 640, 1024])
 @pytest.mark.parametrize("m,n", [(65, 130), (129, 300), (300, 4096), (520, 8200)])
 def test_gemm_ring_edges_4bit(m, n, k):
-    """4-bit weights at few stages and on every output tile: each output equals the same weights' product
+    """4-bit weights at few stages, mostly on 128-row output tiles: each output equals the same weights' product
     in float64 within the accumulation and output rounding (int4: of the bf16-rounded weights)."""
     from scratch_llm_amd.quant import int4_group as i4
     from scratch_llm_amd.quant import nvfp4_mxfp4 as f4

@@ -72,7 +72,7 @@ def _ops():
         return [q.codes, q.s_block] + ([q.s_global.reshape(1)] if hasattr(q, "s_global") else [])
 
     return {
-        "int4": lambda x: i4.quantize_groupwise_int4(x) if x.shape[1] % 128 == 0 else (x,),
+        "int4": lambda x: i4.quantize_groupwise_int4(x, 128 if x.shape[1] % 128 == 0 else 8),
         "int8": lambda x: i8.quantize_symmetric(x, axis=0),
         "int8_affine": lambda x: i8.quantize_affine(x, axis=0),
         "fp8": lambda x: f8.quantize_per_channel(x),
@@ -96,6 +96,32 @@ def test_quantizer_same_on_both_paths(rows, cols, op, dtype):
     f = _ops()[op]
     assert x.data_ptr() % 16 == 0
     _same(f(x), f(_shifted(x)), f"{op} {rows}x{cols}")
+
+
+def _ordinary(rows, cols, dtype, seed):
+    """Finite rows without a huge value, so that one scale for the whole tensor (NVFP4's global one) keeps ordinary
+    quotients: blocks of mixed magnitudes, quotients that underflow, code ties and signed zeros."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(rows, cols, generator=g) * torch.exp2(torch.randint(-12, 1, (rows, max(cols // 8, 1)), generator=g).float()
+                                                          ).repeat_interleave(8, dim=1)[:, :cols]
+    x[:, 1::11] *= 1e-30 if dtype != torch.float16 else 1e-4
+    x[:, 2::13] = -0.0
+    x[-1] = (torch.arange(cols) % 25 - 12) * 0.25  # with 6 as the maximum of each block: every E2M1 tie
+    x[-1, ::8] = 6.0
+    return x.to(dtype).to(DEV)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("op", ["int4", "int8", "int8_affine", "fp8", "mxfp4", "mxfp4_64", "nvfp4", "kv"])
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_quantizer_same_on_both_paths_finite(rows, cols, op, dtype):
+    print_case("quantizer paths, finite", op, f"{rows}x{cols}", str(dtype))
+    x = _ordinary(rows, cols, dtype, rows + cols)
+    f = _ops()[op]
+    out = f(x)
+    _same(out, f(_shifted(x)), f"{op} {rows}x{cols}")
+    if op == "nvfp4":
+        assert bool(torch.isfinite(out[2]).all()) and out[0].unique().numel() >= (4 if cols < 128 else 12)
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 128), (16, 128), (17, 256), (40, 384), (1030, 1152), (33, 4096)])
