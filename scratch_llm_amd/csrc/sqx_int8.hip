@@ -849,26 +849,30 @@ extern "C" int sqx_int8_linear(const uint8_t* wt, const float* scale, const void
   return SQX_OK;
 }
 
-// The launch for 2..64 rows: FP8's, but for the shapes where the GEMV is the faster one. FP8 quantizes its rows in a
-// launch of its own first and its GEMV has no such head start, so its lines are not int8's. From a sweep of bf16
-// activations at 2..64 rows, 512..28672 weight rows and 512..14336 columns (us, GEMV and row-tiled): 512 -> 512 at
-// m = 17 / 64 4.0 / 6.0 and 7.3 / 9.7; 1536 -> 3000 at m = 33 7.0 and 13.3; 4096 -> 16384 at m = 2 13.4 and 16.0;
-// 4096 -> 4096 at m = 24 / 64 9.9 / 18.2 and 10.0 / 15.3.
+// The launch for 2..64 rows: FP8's, but for 257..383 tiles to K = 12288 in one piece of 2 tiles x 8 waves (4096 -> 5120 at
+// m = 16: 12.3 us with the GEMV, 9.9 so) and for the shapes where the call is the faster one with the GEMV. FP8 quantizes
+// its rows in a launch of its own first and its GEMV has no such head start, so its lines are not int8's. A call from
+// Python takes no less than its host time, 13 us with the GEMV and 17.6 us with a split (the workspace and the second
+// launch), so the lines compare max(host, kernel) first and the kernels alone second. From a sweep of bf16 activations at
+// 2..64 rows, 512..28672 weight rows and 512..14336 columns (kernels, us, GEMV and row-tiled): 512 -> 512 at m = 17 / 64
+// 4.0 / 5.9 and 7.5 / 9.8; 1536 -> 3072 at m = 33 6.9 and 13.4; 4096 -> 16384 at m = 2 13.0 and 16.0; 2048 -> 2048 at
+// m = 64 10.4 and 9.7, a split; 4096 -> 4096 at m = 24 / 64 9.8 / 18.2 and 10.1 / 15.4.
 static constexpr GemvUntil kInt8Gemv[] = {
-    { 128, {kG, kG, 24, 24, 20, 24, 20, 10,  8,  7,  4}},
-    { 255, {kG, kG, kG, kG, 22, 24, 20, 16, 16, 16, 11}},
-    { 256, {kG, kG, kG, kG, 22, 24, 20, 12,  8,  8,  6}},
-    { 383, {kG, kG,  0,  0,  0,  0,  0,  8,  6,  6,  6}},
-    { 512, {kG, kG, kG, kG, kG,  5,  4,  3,  2,  2,  0}},
-    { 639, {kG, kG, 10,  3,  3,  3,  5,  3,  3,  3,  3}},
+    { 128, {kG, kG, kG, kG, kG, kG, 28, 22, 18, 11, 10}},
+    { 256, {kG, kG, kG, kG, kG, kG, 28, 22, 16, 16, 11}},
+    { 383, {kG, kG, 24, 24, 12,  5,  5,  3,  3,  2,  0}},
+    { 512, {kG, kG, kG, kG, 20,  5,  4,  3,  2,  2,  0}},
+    { 639, {kG, kG, 10,  3,  3,  3,  3,  3,  3,  3,  3}},
     { 895, {kG, kG,  5,  4,  4,  4,  4,  3,  3,  4,  3}},
-    {1023, {kG, kG,  3,  3,  3,  3,  2,  2,  0,  2,  2}},
+    {1023, {18, 14,  3,  3,  3,  2,  2,  2,  0,  2,  2}},
     {1199, {kG, kG, kG, kG,  5, kG,  7,  5,  3,  3,  2}},
-    {1343, {kG, kG,  4,  4,  2, kG,  4,  4,  3,  3,  2}},
-    {1919, {kG,  5,  2,  2,  2,  3,  2,  2,  2,  2,  0}},
-    {kAllTiles, {kG,  2,  2,  2,  2,  2,  2,  2,  0,  0,  0}}};
+    {1343, {kG, kG,  4,  3,  2, kG,  4,  4,  3,  3,  2}},
+    {1919, {16,  5,  2,  2,  2,  3,  3,  2,  2,  0,  0}},
+    {kAllTiles, { 2,  2,  0,  0,  0,  0,  0,  2,  0,  0,  0}}};
 static SkinnyShape int8_default_shape(int64_t m, int64_t rows, int64_t cols) {
   SkinnyShape sh = skinny64_default_shape(m, rows, cols);
+  const int64_t T = ceil_div(rows, 16);
+  if (m >= 2 && m <= 64 && T > 256 && T < 384 && cols < 12288) sh = SkinnyShape{0, 2, 8, 1, false};
   if (gemv_ahead(kInt8Gemv, m, rows, cols)) sh.gemv = true;
   return sh;
 }

@@ -85,6 +85,8 @@ def test_fp4_launch_shapes(m, variant, tiles, waves, splits):
                                    (20, 1024, 8200), (64, 4096, 1032),
                                    (16, 1030, 10248), (5, 5200, 8200), (64, 4096, 3080), (36, 3000, 8200), (12, 6160, 2056),
                                    (8, 10248, 2056), (48, 14330, 1032), (20, 18440, 2568), (4, 28680, 2568), (64, 32776, 72),
+                                   # 257..383 tiles in one piece, and past them
+                                   (16, 5120, 4104), (33, 4120, 2568), (64, 6120, 12280), (12, 6130, 12296),
                                    # small weights past 64 rows: the last rows of the GEMV, the GEMM's first
                                    (65, 512, 512), (80, 3070, 1536), (104, 1024, 1024), (105, 1024, 1024)])
 def test_int8_rows(m, n, k):
