@@ -1072,49 +1072,59 @@ extern "C" int sqx_fp4_linear(const uint8_t* wt, const uint8_t* st, int fmt, con
 // The library's launch shape for 2..64 rows (16-bit output), from a sweep of MXFP4 weights at 2..63 rows, rotating
 // copies (GEMV -> row-tiled, us): the int4 table but for these, where FP4's cheaper decode (no sums, no group
 // scale) moves the best shape, and the GEMV in place of int4's multi-row GEMV:
-//   1024..4095 tiles, m <= 8   4 tiles x 4 waves (8192 -> 28672 at m = 4 / 8: 33.8 / 43.7 -> 24.8 / 25.7; at 32 rows the
-//                              int4 shape, 109.2 -> 33.0)
-//   384..1023 tiles, K >= 8192 two splits of 4 x 8 to 8 rows, else LDS-staged 2 x 8 in four splits (28672 -> 8192 at
-//                              m = 4 / 32: 38.7 / 110.1 -> 26.7 / 33.7)
-//   640..1023 tiles, shorter K 4 x 8 to 8 rows, LDS-staged 1 x 8 at 17..32 (4096 -> 14336 at m = 4 / 32: 11.0 / 34.2 ->
-//                              9.2 / 13.3)
-// and the GEMV where it is the faster kernel, by format (NVFP4's scales make both kernels decode in more steps). From
-// a sweep of bf16 activations at 2..63 rows, 512..128256 weight rows and 512..14336 columns (us, GEMV and row-tiled;
-// MXFP4, NVFP4): 512 -> 512 at m = 17 4.1 and 6.6, 4.4 and 6.7; 1536 -> 3072 at m = 33 7.1 and 9.6, 7.2 and 10.8;
-// 512 -> 28672 at m = 2 4.2 and 5.8, 5.0 and 6.4; 4096 -> 4096 at m = 17 / 32 7.9 / 10.5 and 8.8 / 10.3, 8.1 / 10.6 and
-// 9.0 / 10.4.
+//   1024..4095 tiles, m <= 8  4 tiles x 4 waves (8192 -> 28672 at m = 4 / 8: 33.8 / 43.7 -> 24.8 / 25.7; at 32 rows
+//                             the int4 shape, 109.2 -> 33.0)
+//   384..1023, K > 16256      two splits of 4 x 8 to 8 rows, else LDS-staged 2 x 8 in four splits (28672 -> 8192 at
+//                             m = 4 / 32: 38.7 / 110.1 -> 26.7 / 33.7)
+//   257..1023, shorter K      to 16 rows 2 (from 513 tiles 4) x 8 in one piece: the reduce of a split is a second
+//                             launch, and one workgroup's k-blocks still hide each other's latency (8192 -> 8192 at
+//                             m = 12: 17.0 -> 11.3; 4096 -> 5120 at m = 16: 10.7 -> 8.2; 4096 -> 14336 at m = 4 / 16:
+//                             11.0 / 18.9 -> 9.2 / 10.6). From 17 rows: at 384 tiles and K > 8064 LDS-staged 2 x 8, in
+//                             four splits to 512 tiles and two above; else at 640 tiles LDS-staged 1 x 8 to 32 rows
+//                             (4096 -> 14336 at m = 32: 34.2 -> 13.3); below 384 tiles 2 x 8 in one piece (4096 ->
+//                             5120 at m = 32: 17.9 -> 11.8) to K = 8064, from 33 rows to K = 4992
+// and the GEMV where the call is the faster one with it, by format (NVFP4's scales make both kernels decode in more
+// steps). A call from Python takes no less than its host time, 13 us with the GEMV and 17.6 us with a split (the
+// workspace and the second launch), so the lines compare max(host, kernel) first and the kernels alone second: a split
+// that saves 1 us of a 10 us kernel would lengthen the call by 4. From a sweep of bf16 activations at 2..63 rows,
+// 512..128256 weight rows and 512..14336 columns (kernels, us, GEMV and row-tiled; MXFP4, NVFP4): 512 -> 512 at m = 17
+// 4.0 and 6.7, 4.2 and 6.8; 1536 -> 3072 at m = 33 7.1 and 9.6, 7.2 and 10.8; 512 -> 28672 at m = 2 4.2 and 5.8, 4.7
+// and 6.4; 4096 -> 4096 at m = 17 / 32 7.9 / 10.5 and 8.9 / 10.4, 8.0 / 10.7 and 9.1 / 10.5.
 static constexpr GemvUntil kMxGemv[] = {
-    {  64, {kG, kG, kG, kG, kG, 20, 14,  8,  8,  8,  6}},
-    { 256, {kG, kG, kG, kG, 20, 18, 16, 11, 11,  8,  6}},
-    { 383, { 0,  0,  0,  0,  0, 12, 12,  7,  6,  0,  0}},
-    { 512, {kG, 18, 10, 10,  7,  5,  0,  3,  0,  0,  0}},
-    { 639, {24, 20, 10, 10,  7,  3,  3,  3,  2,  0,  0}},
-    { 895, {kG, 18, 10,  8,  6,  5,  4,  0,  0,  0,  0}},
-    {1023, {24,  7,  5,  4,  4,  4,  3,  0,  0,  0,  0}},
-    {1343, {kG, 16, 10,  7,  5,  5,  3,  0,  0,  0,  0}},
-    {1919, { 5,  5,  3,  3,  3,  3,  2,  0,  0,  0,  0}},
+    { 128, {kG, kG, kG, kG, kG, kG, kG, 22, 18, 11, 10}},
+    { 256, {kG, kG, kG, kG, kG, kG, kG, 22, 18, 11, 10}},
+    { 383, {kG, 18, 10, 10, 10,  6,  0,  3,  0,  0,  0}},
+    { 512, {kG, 18, 10, 10,  8,  6,  0,  2,  0,  6,  0}},
+    { 639, {24, 14, 10, 10,  7,  3,  3,  3,  2,  0,  0}},
+    { 895, {24, 14, 10,  8,  6,  5,  4,  0,  0,  0,  0}},
+    {1023, {10,  8,  6,  4,  4,  4,  3,  0,  0,  0,  0}},
+    {1343, {kG, 18, 10,  8,  6,  5,  3,  0,  0,  0,  0}},
+    {1919, {16,  5,  3,  3,  3,  3,  2,  0,  0,  0,  0}},
     {3071, { 3,  2,  2,  2,  2,  2,  2,  0,  0,  0,  0}},
-    {kAllTiles, { 2,  2,  0,  0,  0,  0,  0,  0,  0,  0,  0}}};
+    {kAllTiles, {kG,  2,  0,  0,  0,  0,  0,  0,  0,  0,  0}}};
 static constexpr GemvUntil kNvGemv[] = {
-    {  64, {kG, kG, kG, kG, 24, 18, 16,  8,  8,  8,  8}},
-    { 256, {kG, kG, kG, kG, 22, 22, 16, 11, 11,  8,  8}},
-    { 383, {kG, kG,  0,  0,  0,  0,  0, 11,  8,  3,  2}},
-    { 512, {kG, 20, 10, 10,  5,  5,  2,  3,  2,  3,  2}},
-    { 639, {kG, 20, 10, 10,  7,  3,  3, 10, 10,  0,  0}},
-    { 895, {kG, 24, 24, 10,  7,  5,  5,  2,  1,  0,  0}},
-    {1023, {28, 10,  5,  5,  4,  4,  3,  0,  0,  0,  0}},
-    {1199, {kG, kG, kG, 10,  7,  4,  3,  3,  3,  2,  0}},
-    {1343, {kG, kG, kG, kG,  8,  8,  3,  2,  2,  0,  0}},
-    {1919, {kG,  5,  3,  3,  3,  3,  3,  2,  0,  0,  0}},
-    {3071, { 2,  2,  2,  2,  2,  2,  2,  0,  0,  0,  0}},
+    { 128, {kG, kG, kG, kG, kG, kG, kG, 22, 18, 11, 10}},
+    { 256, {kG, kG, kG, kG, kG, kG, kG, 22, 18, 11, 10}},
+    { 383, {24, 14, 10, 10,  8,  6,  0,  3,  0,  0,  0}},
+    { 512, {14, 10,  8,  8,  6,  5,  0,  0,  0,  6,  5}},
+    { 639, {kG, 24, 18, 14, 10, 10,  7, 10, 10,  0,  0}},
+    { 895, {kG, 18, 10, 10,  8,  6,  5,  2,  0,  0,  0}},
+    {1023, {10, 10,  6,  6,  4,  4,  3,  0,  0,  0,  0}},
+    {1199, {kG, kG, kG, 16,  7,  4,  3,  3,  2,  2,  0}},
+    {1343, {kG, kG, kG, kG,  8,  8,  4,  2,  2,  0,  0}},
+    {1919, {kG, 12,  6,  3,  3,  3,  3,  2,  0,  0,  0}},
+    {3071, { 3,  3,  2,  2,  2,  2,  2,  0,  0,  0,  0}},
     {kAllTiles, { 2,  2,  0,  0,  0,  0,  0,  0,  0,  0,  0}}};
 static SkinnyShape fp4_row_tiled_shape(int64_t m, int64_t rows, int64_t cols, bool have_ws) {
   const int64_t T = ceil_div(rows, 16), KB = ceil_div(cols, 128);
   if (m >= 2 && T >= 1024 && T < 4096 && m <= 8) return SkinnyShape{0, 4, 4, 1, false};
-  if (m >= 2 && T >= 384 && T < 1024 && KB >= 64 && have_ws)
-    return m <= 8 ? SkinnyShape{0, 4, 8, 2, false} : SkinnyShape{1, 2, 8, 4, false};
-  if (m >= 2 && T >= 640 && T < 1024 && m <= 8) return SkinnyShape{0, 4, 8, 1, false};
-  if (T >= 640 && T < 1024 && m > 16 && m <= 32) return SkinnyShape{1, 1, 8, 1, false};
+  if (m >= 2 && T > 256 && T < 1024) {
+    if (m <= 16 && (KB < 128 || !have_ws)) return SkinnyShape{0, T <= 512 ? 2 : 4, 8, 1, false};
+    if (T >= 384 && KB >= 64 && have_ws)
+      return m <= 8 ? SkinnyShape{0, 4, 8, 2, false} : SkinnyShape{1, 2, 8, T <= 512 || KB >= 128 ? 4 : 2, false};
+    if (T < 384 && KB < (m <= 32 ? 64 : 40)) return SkinnyShape{0, 2, 8, 1, false};
+    if (T >= 640 && m <= 32) return SkinnyShape{1, 1, 8, 1, false};
+  }
   SkinnyShape sh = skinny_default_shape(m, rows, cols, 128, have_ws);
   if (sh.variant == 2) sh = SkinnyShape{0, 2, 8, 1, true};
   return sh;

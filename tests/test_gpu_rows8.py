@@ -32,7 +32,10 @@ LINEAR = [(2, 16, 32), (3, 1000, 96), (8, 40, 224), (9, 6150, 512), (16, 4096, 1
           (33, 520, 4096), (63, 1024, 8224), (24, 6400, 8192),
           # the row-tiled kernels' side of the choice, for either format
           (6, 28700, 1568), (9, 6150, 2592), (12, 4096, 9248), (4, 10250, 12320), (18, 14400, 544), (40, 28700, 1056),
-          (13, 18000, 2080), (2, 30000, 2592), (36, 5200, 1568), (5, 65552, 96)]
+          (13, 18000, 2080), (2, 30000, 2592), (36, 5200, 1568), (5, 65552, 96),
+          # 257..1023 tiles in one piece and in splits
+          (12, 8200, 8224), (10, 4120, 6176), (7, 10250, 8224), (31, 6200, 8224), (33, 9000, 8096), (36, 5120, 4960),
+          (14, 6160, 16416), (5, 7000, 16288), (16, 4120, 16288)]
 
 
 @pytest.mark.parametrize("fmt", ["mx", "nv"])
