@@ -788,10 +788,12 @@ extern "C" int sqx_quantize_e8m0(const float* v, int64_t n, float* out, sqx_stre
   return SQX_OK;
 }
 
-// Blocks of 16, 32, 64 or 128 elements, all whole, with 16-byte loads and 8-byte stores.
+// Blocks of 16, 32, 64 or 128 elements, all whole, with 16-byte loads and 8-byte stores. A thread per 8 elements: a
+// launch holds fewer than 2^32 threads, so longer tensors keep the thread per block.
 static bool quantize8_fits(const void* x, int64_t n, int64_t block, const uint8_t* codes) {
   return (block == 16 || block == 32 || block == 64 || block == 128) && n % block == 0 &&
-         reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(codes) % 8 == 0;
+         n / 8 <= (int64_t)UINT32_MAX - 256 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(codes) % 8 == 0;
 }
 template <bool NV>
 static void launch_quantize8(const void* x, int dtype, int64_t n, int64_t block, uint8_t* codes, float* s_block,

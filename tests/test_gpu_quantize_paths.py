@@ -227,6 +227,35 @@ def test_int8_many_short_rows(cols):
             _same([y[p]], [i8.w8a8_linear(x[p].contiguous(), w)], f"w8a8 rows {p.start}")
 
 
+def test_mxfp4_as_many_elements_as_a_launch_has_no_threads_for():
+    """2^35 elements: eight a thread would be 2^32 threads, which no launch holds; a block of 128 a thread fits."""
+    from scratch_llm_amd import _lib
+
+    n, block = 1 << 35, 128
+    free, _ = torch.cuda.mem_get_info()
+    if free < 120 << 30:
+        pytest.skip("needs 120 GiB of device memory")
+    print_case("mxfp4 quantize", f"n={n}")
+    lib = _lib.load()
+    x = torch.zeros(n, device=DEV, dtype=torch.bfloat16)
+    codes = torch.full((n,), 7, device=DEV, dtype=torch.uint8)
+    s_block = torch.full((n // block,), 7.0, device=DEV)
+    tail = torch.randn(block, device=DEV, generator=torch.Generator(device=DEV).manual_seed(5)).to(torch.bfloat16)
+    x[-block:] = tail
+    stream = _lib.stream_ptr(x.device)
+    _lib.check(lib.sqx_mxfp4_quantize(x.data_ptr(), _lib.DTYPE_BF16, n, block, codes.data_ptr(), s_block.data_ptr(), None,
+                                      stream), "sqx_mxfp4_quantize")
+    tc, ts = torch.empty(block, device=DEV, dtype=torch.uint8), torch.empty(1, device=DEV)
+    _lib.check(lib.sqx_mxfp4_quantize(tail.data_ptr(), _lib.DTYPE_BF16, block, block, tc.data_ptr(), ts.data_ptr(), None,
+                                      stream), "sqx_mxfp4_quantize")
+    assert torch.equal(codes[-block:], tc) and torch.equal(s_block[-1:], ts)
+    assert bool((s_block[:-1] == s_block[0]).all()) and float(s_block[0]) != 7.0
+    for lo in range(0, n - block, 1 << 31):  # parts small enough for a mask of their own
+        assert not bool(codes[lo:min(lo + (1 << 31), n - block)].any())
+    del x, codes, s_block
+    torch.cuda.empty_cache()
+
+
 # the edge between one workgroup per head and the sliced form (16384 elements a head), rows that split it unevenly,
 # and a head count past one block of the finishing kernel
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
