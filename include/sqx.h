@@ -443,8 +443,10 @@ int sqx_fp4_linear(const uint8_t* wt, const uint8_t* st, int fmt, const float* s
 /* The same product for 1..64 rows with y in act_dtype on the row-tiled decode kernels (as sqx_int4_skinny):
  * variant 0 = waves splitting K (tiles 2 or 4, waves 1..8), 1 = activations staged through LDS (tiles 1, 2 or
  * 4, waves 4 or 8), splits workgroups along K (fp32 partials in ws, added in split order); -1 / 0 = the
- * library's choice, the GEMV included. ws: sqx_fp4_skinny_workspace_bytes(m, rows, cols, splits) bytes. */
+ * library's choice, the GEMV included. ws: sqx_fp4_skinny_workspace_bytes(m, rows, cols, splits) bytes.
+ * sqx_fp4_skinny_gemv: 1 where the choice is the GEMV, so that a caller can call sqx_fp4_linear at once. */
 int64_t sqx_fp4_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits);
+int sqx_fp4_skinny_gemv(int fmt, int64_t m, int64_t rows, int64_t cols);
 int sqx_fp4_skinny(const uint8_t* wt, const uint8_t* st, int fmt, const float* s_global, const void* x,
                    int act_dtype, void* y, const void* bias, int64_t m, int64_t rows, int64_t cols, int variant,
                    int tiles, int waves, int splits, void* ws, int64_t ws_bytes, sqx_stream_t stream);
@@ -591,8 +593,10 @@ int sqx_int8_linear(const uint8_t* wt, const float* scale, const void* x, int ac
                     sqx_stream_t stream);
 /* The same product for 1..64 rows on the row-tiled decode kernel (waves splitting K): tiles (2 or 4) of 16 rows
  * per workgroup, waves 1..8, splits workgroups along K (fp32 partials in ws, added in split order); all 0 = the
- * library's choice, the GEMV included. ws: sqx_int8_skinny_workspace_bytes(m, rows, cols, splits) bytes. */
+ * library's choice, the GEMV included. ws: sqx_int8_skinny_workspace_bytes(m, rows, cols, splits) bytes.
+ * sqx_int8_skinny_gemv: 1 where the choice is the GEMV, so that a caller can call sqx_int8_linear at once. */
 int64_t sqx_int8_skinny_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int splits);
+int sqx_int8_skinny_gemv(int64_t m, int64_t rows, int64_t cols);
 int sqx_int8_skinny(const uint8_t* wt, const float* scale, const void* x, int act_dtype, void* y, const void* bias,
                     int64_t m, int64_t rows, int64_t cols, int tiles, int waves, int splits, void* ws,
                     int64_t ws_bytes, sqx_stream_t stream);

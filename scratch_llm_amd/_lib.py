@@ -127,6 +127,7 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
         [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p],
     ),
     "sqx_fp4_skinny_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i]),
+    "sqx_fp4_skinny_gemv": (_c_i, [_c_i, _c_i64, _c_i64, _c_i64]),
     "sqx_fp4_skinny": (
         _c_i,
         [_c_p, _c_p, _c_i, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_i, _c_i, _c_i, _c_p, _c_i64, _c_p],
@@ -156,6 +157,7 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "sqx_int8_tile": (_c_i, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),
     "sqx_int8_linear": (_c_i, [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_p]),
     "sqx_int8_skinny_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i]),
+    "sqx_int8_skinny_gemv": (_c_i, [_c_i64, _c_i64, _c_i64]),
     "sqx_int8_skinny": (_c_i, [_c_p, _c_p, _c_p, _c_i, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_i, _c_i, _c_p, _c_i64,
                                _c_p]),
     "sqx_int8_gemm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),

@@ -1149,6 +1149,10 @@ extern "C" int64_t sqx_fp4_skinny_workspace_bytes(int64_t m, int64_t rows, int64
   return need;
 }
 
+extern "C" int sqx_fp4_skinny_gemv(int fmt, int64_t m, int64_t rows, int64_t cols) {
+  if (m <= 0 || m > 64 || rows <= 0 || cols <= 0) return 0;
+  return fp4_default_shape(fmt, m, rows, cols, sqx_fp4_skinny_workspace_bytes(m, rows, cols, 0) > 0).gemv;
+}
 extern "C" int sqx_fp4_skinny(const uint8_t* wt, const uint8_t* st, int fmt, const float* s_global, const void* x,
                               int act_dtype, void* y, const void* bias, int64_t m, int64_t rows, int64_t cols,
                               int variant, int tiles, int waves, int splits, void* ws, int64_t ws_bytes,

@@ -884,6 +884,10 @@ extern "C" int64_t sqx_int8_skinny_workspace_bytes(int64_t m, int64_t rows, int6
   return skinny_workspace_bytes(m, rows, skinny_splits(ceil_div(cols, 64), S));
 }
 
+extern "C" int sqx_int8_skinny_gemv(int64_t m, int64_t rows, int64_t cols) {
+  return m > 0 && m <= 64 && rows > 0 && cols > 0 && int8_default_shape(m, rows, cols).gemv;
+}
+
 extern "C" int sqx_int8_skinny(const uint8_t* wt, const float* scale, const void* x, int act_dtype, void* y,
                                const void* bias, int64_t m, int64_t rows, int64_t cols, int tiles, int waves,
                                int splits, void* ws, int64_t ws_bytes, sqx_stream_t stream) {

@@ -288,9 +288,13 @@ GEMM_MIN_M = 65
 
 @functools.lru_cache(maxsize=4096)
 def _rows_workspace(m: int, rows: int, cols: int) -> int:
-    """Workspace bytes of 2..64 rows (0 where the GEMV is chosen), asked of the library once per size: another
-    native call per linear shows at a few rows (2 x 7056 -> 2432: 16.5 us without it, 17.7 with)."""
-    return int(_lib.load().sqx_int8_skinny_workspace_bytes(m, rows, cols, 0))
+    """Workspace bytes of 2..64 rows, -1 where the library chooses the GEMV, asked once per size: another native
+    call per linear shows at a few rows (2 x 7056 -> 2432: 16.5 us without it, 17.7 with), and so do the further
+    arguments of the row-tiled entry (0.5 us a call)."""
+    lib = _lib.load()
+    if lib.sqx_int8_skinny_gemv(m, rows, cols):
+        return -1
+    return int(lib.sqx_int8_skinny_workspace_bytes(m, rows, cols, 0))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -325,8 +329,7 @@ def int8_linear_tiled(x: Tensor, tw: Int8Tiled, bias: Tensor | None = None, k_sl
                                          y.data_ptr(), _lib.ptr(b), m, tw.rows, k, *_lib.ws_args(ws),
                                          _lib.stream_ptr(dev)), "int8_linear")
             return y.reshape(*batch, tw.rows)
-        if 2 <= m < GEMM_MIN_M and k_slices is None:
-            nb = _rows_workspace(m, tw.rows, k)
+        if 2 <= m < GEMM_MIN_M and k_slices is None and (nb := _rows_workspace(m, tw.rows, k)) >= 0:
             ws = torch.empty(nb // 4, dtype=torch.float32, device=dev) if nb > 0 else None
             _lib.check(lib.sqx_int8_skinny(tw.wt.data_ptr(), tw.scale.data_ptr(), x2.data_ptr(), _lib.sqx_dtype(x.dtype),
                                            y.data_ptr(), _lib.ptr(b), m, tw.rows, k, 0, 0, 0, *_lib.ws_args(ws),

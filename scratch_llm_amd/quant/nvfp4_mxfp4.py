@@ -330,10 +330,13 @@ def e4m3_values(codes: Tensor) -> Tensor:
 
 
 @functools.lru_cache(maxsize=4096)
-def _rows_workspace(m: int, rows: int, cols: int) -> int:
-    """Workspace bytes of 2..``GEMM_MIN_M - 1`` rows (0 where the GEMV is chosen), asked of the library once per size:
-    at a few rows another native call per linear shows."""
-    return int(_lib.load().sqx_fp4_skinny_workspace_bytes(m, rows, cols, 0))
+def _rows_workspace(fmt: int, m: int, rows: int, cols: int) -> int:
+    """Workspace bytes of 2..``GEMM_MIN_M - 1`` rows, -1 where the library chooses the GEMV, asked once per size: at a
+    few rows another native call per linear shows, and so do the further arguments of the row-tiled entry."""
+    lib = _lib.load()
+    if lib.sqx_fp4_skinny_gemv(fmt, m, rows, cols):
+        return -1
+    return int(lib.sqx_fp4_skinny_workspace_bytes(m, rows, cols, 0))
 
 
 def fp4_linear_tiled(x: Tensor, tw: FP4Tiled, bias: Tensor | None = None, out_dtype: torch.dtype | None = None,
@@ -386,8 +389,8 @@ def fp4_linear_tiled(x: Tensor, tw: FP4Tiled, bias: Tensor | None = None, out_dt
             _lib.check(lib.sqx_fp4_gemm(tw.wt.data_ptr(), tw.st.data_ptr(), tw.fmt, _lib.ptr(tw.s_global), x2.data_ptr(),
                                         _lib.sqx_dtype(x.dtype), y.data_ptr(), ydt, _lib.ptr(b), m, tw.rows, tw.cols,
                                         *_lib.ws_args(ws), s), "fp4_linear")
-        elif 2 <= m < GEMM_MIN_M and k_slices is None and not yf32:
-            nb = _rows_workspace(m, tw.rows, tw.cols)
+        elif (2 <= m < GEMM_MIN_M and k_slices is None and not yf32
+              and (nb := _rows_workspace(tw.fmt, m, tw.rows, tw.cols)) >= 0):
             ws = torch.empty(nb // 4, dtype=torch.float32, device=dev) if nb > 0 else None
             _lib.check(lib.sqx_fp4_skinny(tw.wt.data_ptr(), tw.st.data_ptr(), tw.fmt, _lib.ptr(tw.s_global), x2.data_ptr(),
                                           _lib.sqx_dtype(x.dtype), y.data_ptr(), _lib.ptr(b), m, tw.rows, tw.cols, -1, 0,

@@ -97,3 +97,20 @@ def test_python_layer_rejects_cpu_tensors():
         int4_group.quantize_groupwise_int4(torch.randn(4, 100))
     with pytest.raises(ValueError, match="2-D"):
         int4_group.quantize_groupwise_int4(torch.randn(128))
+
+
+# the GEMV's classes of row tiles and their edges, rows at the edges of the choice's row ranges
+@pytest.mark.parametrize("rows", [1, 2048, 2049, 4096, 4097, 8192, 14336, 16384, 17000, 28672, 49136, 128256])
+def test_gemv_choice_needs_no_workspace(rows):
+    lib = _lib.load()
+    seen = set()
+    for m in (1, 2, 4, 5, 6, 8, 11, 16, 20, 32, 40, 63, 64):
+        for cols in (64, 512, 1536, 4096, 8192, 14336, 28672):
+            fp4 = [lib.sqx_fp4_skinny_gemv(fmt, m, rows, cols) for fmt in (_lib.FP4_MX, _lib.FP4_NV)]
+            if lib.sqx_int8_skinny_gemv(m, rows, cols):
+                assert lib.sqx_int8_skinny_workspace_bytes(m, rows, cols, 0) == 0
+            if all(fp4):
+                assert lib.sqx_fp4_skinny_workspace_bytes(m, rows, cols, 0) == 0
+            seen.update(fp4, [lib.sqx_int8_skinny_gemv(m, rows, cols)])
+    assert seen <= {0, 1}
+    assert lib.sqx_int8_skinny_gemv(65, rows, 512) == lib.sqx_fp4_skinny_gemv(_lib.FP4_MX, 65, rows, 512) == 0
