@@ -8,6 +8,7 @@ another implementation: a missing library, a CPU tensor or a non-zero status rai
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 from pathlib import Path
@@ -281,9 +282,15 @@ def sqx_dtype(dt: torch.dtype) -> int:
         raise TypeError(f"dtype {dt} is not supported by the HIP kernels") from None
 
 
+@functools.lru_cache(maxsize=4096)
+def _gemm_workspace_bytes(m: int, rows: int, cols: int) -> int:
+    """The GEMMs' workspace query, asked once per size: it evaluates three plans (0.5 to 0.9 us)."""
+    return int(load().sqx_gemm_workspace_bytes(m, rows, cols))
+
+
 def gemm_workspace(m: int, rows: int, cols: int, device: torch.device) -> torch.Tensor | None:
     """fp32 split-K workspace the prefill GEMMs want for this shape (None when they do not split)."""
-    nb = int(load().sqx_gemm_workspace_bytes(m, rows, cols))
+    nb = _gemm_workspace_bytes(m, rows, cols)
     return None if nb <= 0 else torch.empty(nb // 4, dtype=torch.float32, device=device)
 
 

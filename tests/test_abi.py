@@ -114,3 +114,11 @@ def test_gemv_choice_needs_no_workspace(rows):
             seen.update(fp4, [lib.sqx_int8_skinny_gemv(m, rows, cols)])
     assert seen <= {0, 1}
     assert lib.sqx_int8_skinny_gemv(65, rows, 512) == lib.sqx_fp4_skinny_gemv(_lib.FP4_MX, 65, rows, 512) == 0
+
+
+def test_gemm_workspace_is_asked_once_per_size():
+    _lib._gemm_workspace_bytes(1000, 1024, 4096)
+    before = _lib._gemm_workspace_bytes.cache_info()
+    assert _lib._gemm_workspace_bytes(1000, 1024, 4096) == _lib.load().sqx_gemm_workspace_bytes(1000, 1024, 4096)
+    after = _lib._gemm_workspace_bytes.cache_info()
+    assert (after.hits, after.misses) == (before.hits + 1, before.misses)
