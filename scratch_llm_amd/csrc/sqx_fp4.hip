@@ -301,9 +301,10 @@ __global__ __launch_bounds__(256) void amax_partial_kernel(const void* __restric
 #pragma unroll
       for (int e = 0; e < 8; ++e) m = amax_step(m, v[e]);
     }
-  } else
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    m = amax_step(m, load_as_f32(x, dtype, i));
+  } else {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+      m = amax_step(m, load_as_f32(x, dtype, i));
+  }
   red[threadIdx.x] = m;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {

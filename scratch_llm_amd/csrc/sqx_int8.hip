@@ -291,9 +291,9 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
 // stages; 16-byte chunk c of row r lies at slot c ^ (r & 7), so the 16 rows of a fragment read touch distinct
 // banks. w is the MFMA's first operand: a lane's four accumulators are four consecutive columns of one row.
 // The 64-row tile takes grids that 128-row tiles would leave below one workgroup per CU. A form without LDS,
-// one 16 x 16 tile a wave, took 61 us for 256 x 4096 x 4096. The linear with both quantizers, before and now: 132 and
-// 39 us at that size, 536 and 94 us at 2048 x 4096 x 4096, 976 and 192 us at 1024 x 14336 x 4096.
-// (29 us at that size since w8a8_tile_of below and the one quantizer launch.)
+// one 16 x 16 tile a wave, took 61 us for 256 x 4096 x 4096. The linear with both quantizers: 132 us so and 29 now
+// at that size (39 before w8a8_tile_of below and the one quantizer launch); at 2048 x 4096 x 4096 536 and 94 us, at
+// 1024 x 14336 x 4096 976 and 192, both before those two.
 // ----------------------------------------------------------------------------------------------
 typedef int i32x4_t __attribute__((__vector_size__(4 * sizeof(int))));
 

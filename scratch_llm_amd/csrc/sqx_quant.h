@@ -30,7 +30,8 @@ __device__ inline void load8_f32(const void* p, int dtype, int64_t e0, float (&v
 // v / s correctly rounded, for many v and one s, in three operations instead of the dozen of an IEEE fp32
 // division: with r = RN(1/s), q = RN(v r) is within an ulp of v / s, the residual fma(-q, s, v) is exact, and
 // RN(q + residual r) is the correctly rounded quotient (Markstein, "Computation of elementary functions on the
-// IBM RISC System/6000 processor", 1990). The scale's range keeps q and the residual of every quotient of
+// IBM RISC System/6000 processor", 1990; compared with the division on the CPU for every 16-bit mantissa of v against
+// every s, and on 1.2e10 fp32 pairs). The scale's range keeps q and the residual of every quotient of
 // magnitude 2**-20 .. 2**100 away from underflow and overflow; smaller quotients may be off in their last place
 // (and a zero loses its sign), which no code of these quantizers sees. Outside it, and for v that are not
 // finite or huge, the division itself.
