@@ -447,26 +447,31 @@ extern "C" int sqx_mxfp4_gemm_ws(const uint8_t* xt, const uint8_t* xst, const ui
 // 512..28672 weight rows by 512..14336 columns (22 row counts at 22 weights; every tile with every split, int8, MXFP4,
 // NVFP4, symmetric and asymmetric int4). A workgroup fills a CU (its stages take 130 to 160 KiB of LDS; the 8-bit
 // 128 x 256 ring the whole 160), so tiles * S workgroups run in ceil(tiles * S / 256) rounds, each a fixed time
-// (prologue, pipeline fill, epilogue) and ceil(stages / S) stages, which take longer the more CUs are busy. In us,
-// fixed; a stage with one CU busy + what all CUs busy add:
-//                8-bit               MXFP4               NVFP4               int4
-//   256 x 256    3.0; 1.20 + 0.01    3.9; 1.12 + 0.02    3.7; 1.43 + 0.01    3.7; 1.66 + 0.01   fewest bytes and decodes
-//   128 x 256    3.8; 0.68 + 0.11    2.8; 0.72           3.2; 1.07 + 0.05    5.2; 1.08 + 0.01
-//   128 x 128    3.6; 0.40 + 0.08    1.6; 0.48 + 0.08    3.0; 0.65 + 0.09    4.7; 0.58 + 0.11   short m or narrow n
-// A launch takes 4.4 us more, and K splits 3 for the reduce and 1.35 per million outputs and split. The choice is
-// within 0.6 % of the best one over the sweep on average. Without the fixed time, and with MXFP4's stages for
-// NVFP4, wide weights with short rows and NVFP4 went to tiles that are too small: int4 512 -> 28672 at 640 rows 54 us on
-// 128 x 128, 42 on 256 x 256; NVFP4 4096 -> 6144 at 768 rows 77 us on 128 x 256, 61 on 256 x 256 in three splits. The
-// 8-bit column is fitted to int8 and FP8 together (their codes decode in as many steps).
+// (prologue, pipeline fill, epilogue) and ceil(stages / S) stages, both longer the more CUs are busy. In us,
+// fixed with one CU busy + what all CUs busy add; a stage likewise:
+//                8-bit               MXFP4                     NVFP4                     int4
+//   256 x 256    3.0; 1.20 + 0.01    4.4 + 2.4; 1.04 + 0.17    5.4 + 2.2; 1.41 + 0.10    4.2 + 3.2; 1.57 + 0.10
+//   128 x 256    3.8; 0.68 + 0.11    3.8 + 0.6; 0.70 + 0.06    4.4 + 0.7; 1.08 + 0.04    5.5 + 0.3; 0.98 + 0.09
+//   128 x 128    3.6; 0.40 + 0.08    3.4 + 0.8; 0.53           4.6 + 0.7; 0.70 + 0.01    4.4 + 0.6; 0.62 + 0.02
+// Large tiles copy the fewest bytes and decode a weight the fewest times; small ones are for short m or narrow n.
+// K splits add 1 to 3.5 us for the reduce, by tile, and 1.25 (8-bit: 1.35) per million outputs and split. (A launch's
+// own time is the same for all.) The 4-bit formats' rounds and stages are fitted to the unsplit launches alone, which
+// they meet within 2 % on average; the 8-bit column, to the choice, for int8 and FP8 together (their codes decode in as
+// many steps). The choice is within 0.7 % of the best one over the sweep on average. Without the fixed time, and with
+// MXFP4's stages for NVFP4, wide weights with short rows and NVFP4 went to tiles that are too small: int4 512 -> 28672
+// at 640 rows 54 us on 128 x 128, 42 on 256 x 256; NVFP4 4096 -> 6144 at 768 rows 77 us on 128 x 256, 61 on 256 x 256 in
+// three splits. With a fixed time of 3.7 us for int4's 256 x 256, a third round of a few tiles was taken for cheap:
+// 512 -> 26576 at 1119 rows (520 tiles) 70.4 us, 66.1 on 128 x 256.
 DqPlan sqx::dq_plan(int64_t m, int64_t rows, int64_t stages, int fmt) {
   struct Tile {
     int tm, tn;
-    double fixed[4], stage[4], busy[4];
+    double fixed[4], fill[4], stage[4], busy[4], join[4];
   };
   static constexpr Tile kTiles[] = {
-      {256, 256, {3.0, 3.9, 3.7, 3.7}, {1.20, 1.12, 1.43, 1.66}, {0.01, 0.02, 0.01, 0.01}},
-      {128, 256, {3.8, 2.8, 3.2, 5.2}, {0.68, 0.72, 1.07, 1.08}, {0.11, 0.00, 0.05, 0.01}},
-      {128, 128, {3.6, 1.6, 3.0, 4.7}, {0.40, 0.48, 0.65, 0.58}, {0.08, 0.08, 0.09, 0.11}}};
+      {256, 256, {3.0, 4.4, 5.4, 4.2}, {0.0, 2.4, 2.2, 3.2}, {1.20, 1.04, 1.41, 1.57}, {0.01, 0.17, 0.10, 0.10}, {3.0, 1.6, 1.5, 1.1}},
+      {128, 256, {3.8, 3.8, 4.4, 5.5}, {0.0, 0.6, 0.7, 0.3}, {0.68, 0.70, 1.08, 0.98}, {0.11, 0.06, 0.04, 0.09}, {3.0, 3.3, 3.5, 3.3}},
+      {128, 128, {3.6, 3.4, 4.6, 4.4}, {0.0, 0.8, 0.7, 0.6}, {0.40, 0.53, 0.70, 0.62}, {0.08, 0.00, 0.01, 0.02}, {3.0, 2.9, 3.2, 3.4}}};
+  static constexpr double kSum[4] = {1.35e-6, 1.25e-6, 1.25e-6, 1.25e-6};
   const int f = fmt == kDqInt4 ? 3 : fmt == kDqNv ? 2 : fmt == kDqMx ? 1 : 0;
   DqPlan best{256, 256, 1};
   double best_us = 0.0;
@@ -477,8 +482,8 @@ DqPlan sqx::dq_plan(int64_t m, int64_t rows, int64_t stages, int fmt) {
       const int64_t per = ceil_div(stages, S), wgs = tiles * S;
       if (ceil_div(stages, per) != S) continue;  // the last split would be empty
       const double b = wgs >= 256 ? 1.0 : (double)wgs / 256.0;
-      double us = 4.4 + (double)ceil_div(wgs, 256) * (t.fixed[f] + (double)per * (t.stage[f] + t.busy[f] * b));
-      if (S > 1) us += 3.0 + (double)S * (double)m * (double)rows * 1.35e-6;
+      double us = (double)ceil_div(wgs, 256) * (t.fixed[f] + t.fill[f] * b + (double)per * (t.stage[f] + t.busy[f] * b));
+      if (S > 1) us += t.join[f] + (double)S * (double)m * (double)rows * kSum[f];
       if (first || us < best_us) best = DqPlan{t.tm, t.tn, S}, best_us = us, first = false;
     }
   }
